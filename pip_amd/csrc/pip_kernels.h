@@ -29,6 +29,25 @@ namespace PIP_NS {
 // Reduction slots (bit patterns of non-negative doubles; min/max as uint64).
 enum { RED_DT = 0, RED_RHOAC = 1, RED_GMAX = 2, RED_IONPOT = 3, RED_NAN = 4, RED_N = 5 };
 
+// The workgroups of a plain context's launch spread their reductions over up
+// to kRedSlots sets of slots, one per 128-byte line (k_finalize combines
+// them): atomics on one address complete one every ~9.5 ns here, so with a
+// single set the stage that reduces waits for them (four atomics a workgroup
+// bound stage 2 of 16x7 tiles: 360 us at 1024^2, 187 with 16 sets; 16x15
+// tiles, half as many workgroups: 195 -> 185).  red_sets: one set per 64
+// workgroups, as k_finalize pays for each set it reads (0.1 us a step on the
+// smallest grids, where 64 workgroups' atomics take less than a tile).
+constexpr int kRedSlots = 16;
+PIP_HD int red_sets(long long workgroups) {
+  int n = 1;
+  while (n < kRedSlots && 64LL * n < workgroups) n *= 2;
+  return n;
+}
+struct alignas(128) RedSlot {
+  unsigned long long v[RED_N];
+};
+PIP_HD RedSlot red_slot_init();
+
 struct DevScalars {
   double dt;        // dt of the current step (global dt)
   double time;
@@ -67,6 +86,8 @@ struct StageArgs {
                           // tile's cells and their ghost images
   const double* dtc;      // replay kernels: frozen {dt, cmax} of the replayed step
   DevScalars* sc;
+  RedSlot* red;           // reduction slot sets, nred (a power of two) in use
+  int nred;
   int ix, jx, nx, ny;
   long long N;            // plane stride ix*jx
   int istep, t_order, epi;  // epi: 0 none, 1 one cfl round, 2 two rounds + dt reduction
@@ -90,6 +111,13 @@ PIP_HD double as_f64(unsigned long long x) {
   union { double d; unsigned long long u; } c;
   c.u = x;
   return c.d;
+}
+
+PIP_HD RedSlot red_slot_init() {
+  RedSlot r;
+  for (int k = 0; k < RED_N; k++) r.v[k] = 0ull;
+  r.v[RED_DT] = as_u64(1.0e300);
+  return r;
 }
 
 // Store one cell value set (NVT vars) at (ci,cj) and at all its ghost images.
@@ -146,20 +174,23 @@ __device__ __forceinline__ void cfl_rewrite(double* um, double* uh, const StageA
   }
 }
 
-// Workgroup min/max reduction of the dt terms, then one atomic per slot.
-template <int NT>
-__device__ __forceinline__ void block_reduce_store(RoundOut r, int nanflag, bool valid, DevScalars* sc,
+// Workgroup min/max reduction of the dt terms into the slots `red`, one
+// atomic per slot (IR: the rate and ion_pot slots too; they stay 0 without).
+template <int NT, bool IR>
+__device__ __forceinline__ void block_reduce_store(RoundOut r, int nanflag, bool valid, unsigned long long* red,
                                                    double* red_lds) {
   double v0 = valid ? r.dtc : 1.0e300;
   double v1 = valid ? r.rhoac : 0.0;
-  double v2 = valid ? r.gmax : 0.0;
-  double v3 = valid ? r.ratio : 0.0;
+  double v2 = (IR && valid) ? r.gmax : 0.0;
+  double v3 = (IR && valid) ? r.ratio : 0.0;
   int fl = valid ? nanflag : 0;
   for (int off = 32; off > 0; off >>= 1) {
     v0 = dmin(v0, __shfl_xor(v0, off, 64));
     v1 = dmax(v1, __shfl_xor(v1, off, 64));
-    v2 = dmax(v2, __shfl_xor(v2, off, 64));
-    v3 = dmax(v3, __shfl_xor(v3, off, 64));
+    if (IR) {
+      v2 = dmax(v2, __shfl_xor(v2, off, 64));
+      v3 = dmax(v3, __shfl_xor(v3, off, 64));
+    }
     fl |= __shfl_xor(fl, off, 64);
   }
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -168,8 +199,10 @@ __device__ __forceinline__ void block_reduce_store(RoundOut r, int nanflag, bool
   if (lane == 0) {
     red_lds[wid * 5 + 0] = v0;
     red_lds[wid * 5 + 1] = v1;
-    red_lds[wid * 5 + 2] = v2;
-    red_lds[wid * 5 + 3] = v3;
+    if (IR) {
+      red_lds[wid * 5 + 2] = v2;
+      red_lds[wid * 5 + 3] = v3;
+    }
     red_lds[wid * 5 + 4] = (double)fl;
   }
   __syncthreads();
@@ -177,15 +210,19 @@ __device__ __forceinline__ void block_reduce_store(RoundOut r, int nanflag, bool
     for (int w = 1; w < NW; w++) {
       v0 = dmin(v0, red_lds[w * 5 + 0]);
       v1 = dmax(v1, red_lds[w * 5 + 1]);
-      v2 = dmax(v2, red_lds[w * 5 + 2]);
-      v3 = dmax(v3, red_lds[w * 5 + 3]);
+      if (IR) {
+        v2 = dmax(v2, red_lds[w * 5 + 2]);
+        v3 = dmax(v3, red_lds[w * 5 + 3]);
+      }
       fl |= (int)red_lds[w * 5 + 4];
     }
-    atomicMin(&sc->red[RED_DT], as_u64(v0));
-    atomicMax(&sc->red[RED_RHOAC], as_u64(v1));
-    atomicMax(&sc->red[RED_GMAX], as_u64(v2));
-    atomicMax(&sc->red[RED_IONPOT], as_u64(v3));
-    if (fl) atomicOr(&sc->red[RED_NAN], 1ull);
+    atomicMin(&red[RED_DT], as_u64(v0));
+    atomicMax(&red[RED_RHOAC], as_u64(v1));
+    if (IR) {
+      atomicMax(&red[RED_GMAX], as_u64(v2));
+      atomicMax(&red[RED_IONPOT], as_u64(v3));
+    }
+    if (fl) atomicOr(&red[RED_NAN], 1ull);
   }
 }
 
@@ -486,7 +523,7 @@ __global__ void __launch_bounds__(NT, 2) k_stage(StageArgs a) {
   bool valid = stage_tile<NDIM, NV, IR, EXT, TX, TY, NT, MODE>(a, dt, cmax, epi, i0, j0, smem, r, nanflag);
   if (!REPLAY && a.epi >= 1) {
     __syncthreads();
-    block_reduce_store<NT>(r, nanflag, valid, sc, smem);
+    block_reduce_store<NT, IR>(r, nanflag, valid, a.red[blockIdx.x & (a.nred - 1)].v, smem);
   }
 }
 
@@ -726,7 +763,7 @@ __global__ void __launch_bounds__(NT, 3) k_stage2p(StageArgs a) {
   }
   if (!REPLAY && a.epi >= 1) {
     __syncthreads();
-    block_reduce_store<NT>(r, nanflag, valid, sc, smem);
+    block_reduce_store<NT, IR>(r, nanflag, valid, a.red[blockIdx.x & (a.nred - 1)].v, smem);
   }
 }
 
@@ -740,7 +777,8 @@ struct RoundArgs {
   double* gm_ion;
   double* arb_heat;
   const double* ion_pot;
-  DevScalars* sc;
+  RedSlot* red;
+  int nred;
   int ix, jx, nx, ny;
   long long N;
   int do_ir, init_arb, do_cfl, read_rates, do_col;
@@ -801,7 +839,7 @@ __global__ void __launch_bounds__(256) k_round(RoundArgs a) {
 #pragma unroll
     for (int n = 0; n < NVT; n++) a.U[n * N + k] = u[n];
   }
-  if (a.do_cfl) block_reduce_store<256>(r, nanflag, inb, a.sc, red_lds);
+  if (a.do_cfl) block_reduce_store<256, IR>(r, nanflag, inb, a.red[blockIdx.x & (a.nred - 1)].v, red_lds);
 }
 
 // Ghost fill by the composite x-then-y map (Boundary_rot.f90:34-125).
@@ -834,6 +872,8 @@ __global__ void __launch_bounds__(256) k_bnd(double* U, int nvt, int ix, int jx,
 // hist[2 hist_k], hist[2 hist_k + 1], as k_record_dt would write them.
 struct FinArgs {
   DevScalars* sc;
+  RedSlot* red;
+  int nred;
   int mode, into_global, flag_ir, flag_ir_type, flag_divb, pip_imp;
   double safety, dxyz_min, pip_imp_factor;
   double* hist;
@@ -845,31 +885,42 @@ __device__ __forceinline__ void record_dt(const DevScalars* sc, double* hist, in
   hist[2 * k + 1] = sc->cmax;
 }
 
-__global__ void k_finalize(FinArgs f) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ void __launch_bounds__(64) k_finalize(FinArgs f) {
   DevScalars* sc = f.sc;
   if (f.mode == 1 && !sc->active) {
-    if (f.hist) record_dt(sc, f.hist, f.hist_k);
+    if (f.hist && threadIdx.x == 0) record_dt(sc, f.hist, f.hist_k);
     return;
   }
+  // each of the first lanes takes one slot set and resets it
+  if ((int)threadIdx.x >= f.nred) return;
+  RedSlot rs = f.red[threadIdx.x];
+  f.red[threadIdx.x] = red_slot_init();
+  const int nan = __builtin_amdgcn_ballot_w64(rs.v[RED_NAN] != 0ull) != 0ull;
+  auto lo = [](unsigned long long a, unsigned long long b) { return a < b ? a : b; };
+  auto hi = [](unsigned long long a, unsigned long long b) { return a > b ? a : b; };
+  for (int off = f.nred / 2; off > 0; off >>= 1) {  // as the slots' atomics would
+    rs.v[RED_DT] = lo(rs.v[RED_DT], __shfl_xor(rs.v[RED_DT], off, 64));
+    rs.v[RED_RHOAC] = hi(rs.v[RED_RHOAC], __shfl_xor(rs.v[RED_RHOAC], off, 64));
+    if (f.flag_ir >= 1) {
+      rs.v[RED_GMAX] = hi(rs.v[RED_GMAX], __shfl_xor(rs.v[RED_GMAX], off, 64));
+      rs.v[RED_IONPOT] = hi(rs.v[RED_IONPOT], __shfl_xor(rs.v[RED_IONPOT], off, 64));
+    }
+  }
+  const double rdt = as_f64(rs.v[RED_DT]), rhoac = as_f64(rs.v[RED_RHOAC]);
+  const double gmax = as_f64(rs.v[RED_GMAX]), ratio = as_f64(rs.v[RED_IONPOT]);
+  if (threadIdx.x != 0) return;
   if (f.mode == 1) sc->ion_pot_valid = 1;  // source_PIP ran in this step
-  double dttemp = dmin(10.0, as_f64(sc->red[RED_DT]));
+  double dttemp = dmin(10.0, rdt);
   // cfl_pn_col (Scheme_rot.f90:305-313)
-  if (f.pip_imp == 1) dttemp = dmin(dttemp, f.pip_imp_factor / as_f64(sc->red[RED_RHOAC]));
-  else dttemp = dmin(dttemp, dmin(f.safety, 0.3) / as_f64(sc->red[RED_RHOAC]));
+  if (f.pip_imp == 1) dttemp = dmin(dttemp, f.pip_imp_factor / rhoac);
+  else dttemp = dmin(dttemp, dmin(f.safety, 0.3) / rhoac);
   if (f.flag_ir >= 1) {
-    dttemp = dmin(dttemp, dmin(f.safety, 0.1) / dmax(as_f64(sc->red[RED_GMAX]), 1.0e-5));
+    dttemp = dmin(dttemp, dmin(f.safety, 0.1) / dmax(gmax, 1.0e-5));
     if (f.flag_ir_type == 0) {
-      double mx = sc->ion_pot_valid ? as_f64(sc->red[RED_IONPOT]) : 0.0;
+      double mx = sc->ion_pot_valid ? ratio : 0.0;
       dttemp = dmin(dttemp, f.safety / dmax(mx, 1.0e-5));
     }
   }
-  int nan = (int)(sc->red[RED_NAN] != 0ull);
-  sc->red[RED_DT] = as_u64(1.0e300);
-  sc->red[RED_RHOAC] = 0ull;
-  sc->red[RED_GMAX] = 0ull;
-  sc->red[RED_IONPOT] = 0ull;
-  sc->red[RED_NAN] = 0ull;
   sc->dt_out = dttemp;
   if (f.mode == 0 || f.mode == 2) {
     if (f.into_global) sc->dt = dttemp;
@@ -1020,6 +1071,8 @@ __device__ __forceinline__ StageArgs ens_stage_args(const EnsArgs& e, const EnsM
   a.Vout = nullptr;
   a.dtc = nullptr;
   a.sc = nullptr;
+  a.red = nullptr;
+  a.nred = 0;
   a.ix = M.ix;
   a.jx = 1;
   a.nx = M.nx;
@@ -1265,7 +1318,7 @@ __global__ void __launch_bounds__(TX) k_lock_stage(EnsArgs e, DevScalars* scs, c
   const bool valid = stage_tile<1, 8, false, false, TC, 1, TX>(a, dt, 0.0, epi, t.i0, 0, smem, r, nanflag);
   if (ISTEP == 2) {
     __syncthreads();
-    block_reduce_store<TX>(r, nanflag, valid, sc, smem);
+    block_reduce_store<TX, false>(r, nanflag, valid, sc->red, smem);
   }
 }
 
@@ -1418,7 +1471,7 @@ __global__ void __launch_bounds__(kEns2NT, 2) k_lock_stage2(EnsArgs e, DevScalar
                                                                                r, nanflag);
   if (ISTEP == 2) {
     __syncthreads();
-    block_reduce_store<kEns2NT>(r, nanflag, valid, sc, smem);
+    block_reduce_store<kEns2NT, false>(r, nanflag, valid, sc->red, smem);
   }
 }
 

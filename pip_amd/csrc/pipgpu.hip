@@ -85,7 +85,9 @@ struct pip_ctx {
   double* arb_heat = nullptr;
   double* ion_pot = nullptr;
   double* Ub = nullptr;  // implicit collisions: updated stage base
-  DevScalars* sc = nullptr;
+  DevScalars* sc = nullptr;  // with the reduction slots after it (CtxScalars)
+  RedSlot* red = nullptr;
+  int nred = 1;              // slot sets in use (red_sets)
   hipStream_t stream = nullptr;
   int tx = 16, ty = 15;
   int xcd_remap = 0;  // contiguous tile ranges per XCD (autotuned)
@@ -115,16 +117,21 @@ struct pip_ctx {
 
 static void build_bnd(pip_ctx* c) { c->bnd = make_bnd(c->cfg.flag_bnd, c->cfg.ndim, c->nv, c->cfg.flag_divb); }
 
-static DevScalars host_scalars_init() {
-  DevScalars s;
+// The scalars of a context and its reduction slots, one device block.
+struct CtxScalars {
+  DevScalars sc;
+  RedSlot red[kRedSlots];
+};
+static_assert(sizeof(DevScalars) == 128, "the slots start on a line of their own");
+
+static CtxScalars host_scalars_init() {
+  CtxScalars s;
   memset(&s, 0, sizeof(s));
-  s.dt = 0.0;
-  s.time = 0.0;
-  s.cmax = 0.0;
-  s.tend = 1.0e300;
-  s.red[RED_DT] = as_u64(1.0e300);
-  s.nmax = (long long)1 << 62;
-  s.active = 1;
+  s.sc.tend = 1.0e300;
+  s.sc.red[RED_DT] = as_u64(1.0e300);
+  s.sc.nmax = (long long)1 << 62;
+  s.sc.active = 1;
+  for (auto& r : s.red) r = red_slot_init();
   return s;
 }
 
@@ -146,6 +153,8 @@ static StageArgs stage_args(pip_ctx* c, int istep, const double* Uin, const doub
   a.Vout = nullptr;
   a.dtc = nullptr;
   a.sc = c->sc;
+  a.red = c->red;
+  a.nred = c->nred;
   a.ix = c->cfg.ix;
   a.jx = c->cfg.jx;
   a.nx = c->nx;
@@ -278,7 +287,8 @@ static RoundArgs round_args(pip_ctx* c, int do_ir, int init_arb, int do_cfl, int
   r.gm_ion = c->gm_ion;
   r.arb_heat = c->arb_heat;
   r.ion_pot = ion_pot;
-  r.sc = c->sc;
+  r.red = c->red;
+  r.nred = c->nred;
   r.ix = c->cfg.ix;
   r.jx = c->cfg.jx;
   r.nx = c->nx;
@@ -313,6 +323,8 @@ static int launch_round(pip_ctx* c, const RoundArgs& r) {
 static int launch_finalize(pip_ctx* c, int mode, int into_global, double* hist = nullptr, int hist_k = 0) {
   FinArgs f;
   f.sc = c->sc;
+  f.red = c->red;
+  f.nred = c->nred;
   f.hist = hist;
   f.hist_k = hist_k;
   f.mode = mode;
@@ -426,6 +438,9 @@ int pip_create(const pip_cfg* cfg, pip_ctx** out) {
   c->dxyz_min = dmin(dmin(cfg->dx, dy), dz);
   c->gmin_safety = cfg->safety * c->dxyz_min;
   build_bnd(c);
+  // by the 16x15 (255-cell) tiles, whatever tile is set: the set count is fixed
+  // for the context
+  c->nred = red_sets(cfg->ndim == 2 ? (long long)((c->nx + 15) / 16) * ((c->ny + 14) / 15) : (c->nx + 254) / 255);
   hipError_t e;
   size_t bytes = sizeof(double) * (size_t)c->N;
   auto cleanup = [&](const char* what) {
@@ -450,8 +465,9 @@ int pip_create(const pip_cfg* cfg, pip_ctx** out) {
     if ((e = hipMemset(c->arb_heat, 0, bytes)) != hipSuccess) return cleanup("hipMemset");
     if ((e = hipMemset(c->ion_pot, 0, bytes)) != hipSuccess) return cleanup("hipMemset");
   }
-  if ((e = hipMalloc(&c->sc, sizeof(DevScalars))) != hipSuccess) return cleanup("hipMalloc scalars");
-  DevScalars hs = host_scalars_init();
+  if ((e = hipMalloc(&c->sc, sizeof(CtxScalars))) != hipSuccess) return cleanup("hipMalloc scalars");
+  c->red = reinterpret_cast<CtxScalars*>(c->sc)->red;
+  CtxScalars hs = host_scalars_init();
   if ((e = hipMemcpy(c->sc, &hs, sizeof(hs), hipMemcpyHostToDevice)) != hipSuccess) return cleanup("hipMemcpy");
   if ((e = hipMemset(c->U, 0, bytes * c->nvt)) != hipSuccess) return cleanup("hipMemset");
   if ((e = hipMemset(c->U1, 0, bytes * c->nvt)) != hipSuccess) return cleanup("hipMemset");
@@ -535,7 +551,7 @@ int pip_cfl(pip_ctx* c, double* dt, int into_global) {
 
 int pip_prologue(pip_ctx* c, double* dt) {
   if (!c) return fail(PIP_ERR_ARG, "null context");
-  DevScalars hs = host_scalars_init();
+  CtxScalars hs = host_scalars_init();
   HIPCHK(hipMemcpyAsync(c->sc, &hs, sizeof(hs), hipMemcpyHostToDevice, c->stream));
   // set_IR fixes arb_heat on its first call of a fresh run only
   // (PIP_rot.f90:219-229: nout = 0 and no restart)
