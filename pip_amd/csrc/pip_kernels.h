@@ -6,7 +6,8 @@
 //
 // One launch of k_stage performs one SSP-RK stage for both fluids on a
 // TX x TY tile of interior cells per workgroup:
-//   load  : (TX+4)x(TY+4) cells -> primitives in LDS (u2v_*, HLL_rot.f90:1136-1186)
+//   load  : the TX x TY cells and the two-deep ring around them (no corners)
+//           -> primitives in LDS (u2v_*, HLL_rot.f90:1136-1186)
 //   x     : (TX+1)*TY faces: minmod MUSCL + HLLD, then minmod MUSCL + HLLC
 //           (one fluid at a time, so the neutral face states are not live
 //           while HLLD runs) -> flux tile in LDS
@@ -266,47 +267,76 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, double dt, double
   const long long N = a.N;
   const int ix = a.ix;
 
-  // ---- load halo tile -> primitives in LDS
-  for (int c = tid; c < HX * HY; c += NT) {
-    int hx = c % HX, hy = c / HX;
-    int gi = i0 + hx, gj = (NDIM == 2) ? j0 + hy : 0;
-    if (gi < a.ix && gj < a.jx) {
-      long long o = (long long)gj * ix + gi;
-      double um[NV], uh[5];
+  // ---- the tile's cells and the ring of halo cells its stencils reach (two
+  // deep, no corners) -> primitives in LDS.  Each thread loads its own cell
+  // and keeps it for the cell phase; the first NR threads also convert a ring
+  // cell, whose loads are issued with the first ones.  The waves spend a third
+  // of their cycles waiting, mostly on loads: against a loop over the (TX+4) x
+  // (TY+4) cells with the own cell read again after the x faces, a step of
+  // Orszag-Tang 1024^2 went from 349 to 330 us, of KH + IR 2048^2 from 1.53
+  // to 1.49 ms (16x15 tiles: 364 instead of 380 cells in 6 instead of 7 waves).
+  const int ti = tid % TX, tj = tid / TX;
+  const int ci = i0 + ti + 2, cj = (NDIM == 2) ? j0 + tj + 2 : 0;
+  const bool valid = (tid < TX * TY) && (i0 + ti < a.nx) && (j0 + tj < a.ny);
+  const long long oc = (long long)cj * ix + ci;
+  constexpr int NRX = (NDIM == 2) ? 4 * TX : 0;  // ring cells above and below
+  constexpr int NR = NRX + 4 * TY;               // ... and at the sides
+  // past the grid's edge a tile still needs the ghost cells there
+  const bool inside = (tid < TX * TY) && ci < a.ix && cj < a.jx;
+  // (in 2-D; 1-D tiles read it again, as the 26 registers across the solvers
+  // would cost the third workgroup of a CU)
+  constexpr bool KEEP = NDIM == 2;
+  double raw[NVT];
+  if (inside) {
 #pragma unroll
-      for (int n = 0; n < NV; n++) um[n] = a.Uin[n * N + o];
+    for (int n = 0; n < NVT; n++) raw[n] = a.Uin[n * N + oc];
+  }
+  auto convert = [&](const double* u, int hx, int hy, double* v) {
+    double um[NV], uh[5];
 #pragma unroll
-      for (int n = 0; n < 5; n++) uh[n] = a.Uin[(NV + n) * N + o];
-      if (EXT && col_type(a.ph) >= 1) {  // set_collisional's get_Te_* rewrite E (PIP_rot.f90:57-58)
-        double pr, te;
-        getpr_mhd(um, pr, te, a.ph);
-        getpr_hd(uh, pr, te, a.ph);
-      }
-      if (IR) {  // set_IR of set_coefficients(.,1) rewrites E (Solver_rot.f90:111-113)
-        double pr, te;
-        getpr_hd(uh, pr, te, a.ph);
-        getpr_mhd(um, pr, te, a.ph);
-      }
-      double vm[NV], vh[5];
-      u2v_mhd<NV>(um, vm, a.ph);
-      u2v_hd(uh, vh, a.ph);
+    for (int n = 0; n < NV; n++) um[n] = u[n];
 #pragma unroll
-      for (int n = 0; n < NV; n++) V[(n * HY + hy) * HX + hx] = vm[n];
-#pragma unroll
-      for (int n = 0; n < 5; n++) V[((NV + n) * HY + hy) * HX + hx] = vh[n];
-      if (MODE != STAGE_PLAIN && a.Vout && hx >= 2 && hx < TX + 2 && gi < a.nx + 2 &&
-          (NDIM == 1 || (hy >= 2 && hy < TY + 2 && gj < a.ny + 2))) {
-        // a cell of this tile: its primitives and their ghost images (u2v
-        // commutes with the boundary sign maps: v = m / rho, the pressure
-        // takes squares)
-        double vv[NVT];
-#pragma unroll
-        for (int n = 0; n < NV; n++) vv[n] = vm[n];
-#pragma unroll
-        for (int n = 0; n < 5; n++) vv[NV + n] = vh[n];
-        store_cell<NDIM, NVT>(a.Vout, N, ix, a.jx, gi, gj, vv, a.bnd);
-      }
+    for (int n = 0; n < 5; n++) uh[n] = u[NV + n];
+    if (EXT && col_type(a.ph) >= 1) {  // set_collisional's get_Te_* rewrite E (PIP_rot.f90:57-58)
+      double pr, te;
+      getpr_mhd(um, pr, te, a.ph);
+      getpr_hd(uh, pr, te, a.ph);
     }
+    if (IR) {  // set_IR of set_coefficients(.,1) rewrites E (Solver_rot.f90:111-113)
+      double pr, te;
+      getpr_hd(uh, pr, te, a.ph);
+      getpr_mhd(um, pr, te, a.ph);
+    }
+    u2v_mhd<NV>(um, v, a.ph);
+    u2v_hd(uh, v + NV, a.ph);
+#pragma unroll
+    for (int n = 0; n < NVT; n++) V[(n * HY + hy) * HX + hx] = v[n];
+  };
+  for (int r = tid; r < NR; r += NT) {
+    int hx, hy;
+    if (r < NRX) {
+      const int k = r / TX;
+      hy = k < 2 ? k : TY + k;
+      hx = 2 + r % TX;
+    } else {
+      const int k = (r - NRX) % 4;
+      hy = OY + (r - NRX) / 4;
+      hx = k < 2 ? k : TX + k;
+    }
+    const int gi = i0 + hx, gj = (NDIM == 2) ? j0 + hy : 0;
+    if (gi < a.ix && gj < a.jx) {
+      double u[NVT], v[NVT];
+#pragma unroll
+      for (int n = 0; n < NVT; n++) u[n] = a.Uin[n * N + (long long)gj * ix + gi];
+      convert(u, hx, hy, v);
+    }
+  }
+  if (inside) {
+    double v[NVT];
+    convert(raw, ti + 2, tj + OY, v);
+    // the cell's primitives and their ghost images (u2v commutes with the
+    // boundary sign maps: v = m / rho, the pressure takes squares)
+    if (MODE != STAGE_PLAIN && a.Vout && valid) store_cell<NDIM, NVT>(a.Vout, N, ix, a.jx, ci, cj, v, a.bnd);
   }
   __syncthreads();
 
@@ -352,20 +382,16 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, double dt, double
   __syncthreads();
 
   // ---- own cell: sources and x update
-  const int ti = tid % TX, tj = tid / TX;
-  const int ci = i0 + ti + 2, cj = (NDIM == 2) ? j0 + tj + 2 : 0;
-  const bool valid = (tid < TX * TY) && (i0 + ti < a.nx) && (j0 + tj < a.ny);
   double un[NVT];
   double Sm[5], Sh[5];
   double ion_pot = 0.0;
   double acc = a.col;
-  const long long oc = (long long)cj * ix + ci;
   if (valid) {
     double um[NV], uh[5];
 #pragma unroll
-    for (int n = 0; n < NV; n++) um[n] = a.Uin[n * N + oc];
+    for (int n = 0; n < NV; n++) um[n] = KEEP ? raw[n] : a.Uin[n * N + oc];
 #pragma unroll
-    for (int n = 0; n < 5; n++) uh[n] = a.Uin[(NV + n) * N + oc];
+    for (int n = 0; n < 5; n++) uh[n] = KEEP ? raw[NV + n] : a.Uin[(NV + n) * N + oc];
     if (a.ac) acc = a.ac[oc];
     if (EXT && col_type(a.ph) >= 1) {  // set_collisional (PIP_rot.f90:44-97), before set_IR
       acc = set_col_cell(um, uh, a.col, a.ph);
@@ -498,8 +524,9 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, double dt, double
 // ------------------------------------------------------------ stage kernel
 // One workgroup per tile.  The look-ahead round of the fused step (epi=2)
 // is skipped on the loop's last step (sc->last), as main.f90 ends there.
+// 1-D tiles leave room for three workgroups per CU, 2-D tiles for two.
 template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, int NT, int MODE>
-__global__ void __launch_bounds__(NT, 2) k_stage(StageArgs a) {
+__global__ void __launch_bounds__(NT, NDIM == 1 ? 3 : 2) k_stage(StageArgs a) {
   extern __shared__ double smem[];
   DevScalars* sc = a.sc;
   constexpr bool REPLAY = (MODE == STAGE_REPLAY);
@@ -1280,7 +1307,7 @@ __global__ void __launch_bounds__(TX) k_lock_start(EnsArgs e, DevScalars* scs) {
 // workgroup; p = k & 1.  Stage 1 with apply_end first applies step k-1's
 // end; stage 2 carries the cfl rounds and reduces into the member's slots.
 template <int TX, int ISTEP>
-__global__ void __launch_bounds__(TX) k_lock_stage(EnsArgs e, DevScalars* scs, const LockTile* tiles, int p,
+__global__ void __launch_bounds__(TX, 3) k_lock_stage(EnsArgs e, DevScalars* scs, const LockTile* tiles, int p,
                                                    int apply_end) {
   extern __shared__ double smem[];
   constexpr int TC = TX - 1;
