@@ -191,6 +191,7 @@ PIP_HD double ppow(double x, double y) {
 struct Phys {
   double gm, ro_lim, pr_lim, safety;
   double T0, n0, beta, t_ir;
+  double rgm1;       // 1 / (gm - 1), for the quotients by gm - 1 of pip_riemann.h
   int flag_col;      // 1 constant alpha; 2..7 set_collisional (parity selects the IR normalisation)
   int flag_ir;       // 0 or 3
   int flag_ir_type;  // 0, 1, 2

@@ -422,6 +422,7 @@ int pip_create(const pip_cfg* cfg, pip_ctx** out) {
   c->ny = (cfg->ndim == 2) ? cfg->jx - 4 : 1;
   c->N = (long long)cfg->ix * cfg->jx;
   c->ph.gm = cfg->gm;
+  c->ph.rgm1 = 1.0 / (cfg->gm - 1.0);
   c->ph.ro_lim = cfg->ro_lim;
   c->ph.pr_lim = cfg->pr_lim;
   c->ph.safety = cfg->safety;
@@ -1545,6 +1546,7 @@ int pip_ens_create(const pip_cfg* base, const pip_ens_member* members, int n, pi
   e->twod = twod;
   e->nvt = base->nvar_m + 5;
   e->ph.gm = base->gm;
+  e->ph.rgm1 = 1.0 / (base->gm - 1.0);
   e->ph.ro_lim = base->ro_lim;
   e->ph.pr_lim = base->pr_lim;
   e->ph.safety = base->safety;
