@@ -140,7 +140,8 @@ int pip_set_two_pass(pip_ctx *ctx, int stage_mask);
 #define PIP_ARITH_RELAXED 1
 int pip_set_arith(pip_ctx *ctx, int mode);
 /* 1: map workgroups to tiles so that each of the 8 XCDs gets a contiguous
- * range of tiles (neighbouring halos in one L2); 0: row-major (autotuner). */
+ * range of tiles (neighbouring halos in one L2; a 2-D context starts with
+ * it); 0: row-major (autotuner). */
 int pip_set_xcd_remap(pip_ctx *ctx, int on);
 /* Average device time (ms) of the last timed enqueue of the dominant kernel;
  * measured with hipEvents on the context's stream. */
