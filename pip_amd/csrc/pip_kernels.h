@@ -22,6 +22,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "pip_bnd.h"
 #include "pip_phys.h"
 #include "pip_riemann.h"
@@ -36,13 +38,14 @@ enum { RED_DT = 0, RED_RHOAC = 1, RED_GMAX = 2, RED_IONPOT = 3, RED_NAN = 4, RED
 // them): atomics on one address complete one every ~9.5 ns here, so with a
 // single set the stage that reduces waits for them (four atomics a workgroup
 // bound stage 2 of 16x7 tiles: 360 us at 1024^2, 187 with 16 sets; 16x15
-// tiles, half as many workgroups: 195 -> 185).  red_sets: one set per 64
-// workgroups, as k_finalize pays for each set it reads (0.1 us a step on the
-// smallest grids, where 64 workgroups' atomics take less than a tile).
+// tiles, half as many workgroups: 195 -> 185).  red_sets: one set per 16
+// workgroups, whose atomics take 0.6 us (with one per 64, stage 2 of KH + IR
+// 160^2, whose 230 workgroups end together, took 20.3 instead of 16.8 us);
+// k_finalize pays 0.1 us a step for 16 sets.
 constexpr int kRedSlots = 16;
 PIP_HD int red_sets(long long workgroups) {
   int n = 1;
-  while (n < kRedSlots && 64LL * n < workgroups) n *= 2;
+  while (n < kRedSlots && 16LL * n < workgroups) n *= 2;
   return n;
 }
 struct alignas(128) RedSlot {
@@ -562,6 +565,260 @@ __global__ void __launch_bounds__(NT, NDIM == 1 ? 3 : 2) k_stage(StageArgs a) {
   RoundOut r;
   int nanflag;
   bool valid = stage_tile<NDIM, NV, IR, EXT, TX, TY, NT, MODE>(a, dt, cmax, epi, i0, j0, smem, r, nanflag);
+  if (!REPLAY && a.epi >= 1) {
+    __syncthreads();
+    block_reduce_store<NT, IR>(r, nanflag, valid, a.red[blockIdx.x & (a.nred - 1)].v, smem);
+  }
+}
+
+// ------------------------------------------------------ split stage tile
+// The stage of stage_tile for grids that leave CUs idle, where a stage takes as
+// long as one tile's chain of dependent operations: each tile spreads over eight
+// waves (1-D: four), one workgroup per CU.  The waves split into jobs that run
+// side by side: the plasma and the neutrals and, with DIRS, each one's x and y
+// faces.  The x-face waves load, convert and update the tile's cells of their
+// fluid, the y-face waves convert the ring (without DIRS one job does all of a
+// fluid); the neutrals' waves, whose solver is the shorter, also form the
+// sources while the plasma's faces run and hand its part over through shared
+// memory.  Every value comes from the operations of stage_tile, in its order.
+template <int NDIM, int NV, int TX, int TY, bool DIRS>
+struct SplitGeom {
+  static constexpr int NVT = NV + 5;
+  static constexpr int NT = (NDIM == 2) ? 512 : 256;
+  static constexpr int NB = DIRS ? NT / 4 : NT / 2;  // threads of a job
+  static constexpr int HX = TX + 4;
+  static constexpr int HY = (NDIM == 2) ? TY + 4 : 1;
+  static constexpr int NC = TX * TY;
+  static constexpr int NFX = (TX + 1) * TY;
+  static constexpr int NFY = (NDIM == 2) ? TX * (TY + 1) : 0;
+  static constexpr int NX = 17;  // handed from the neutrals to the plasma, per cell
+  static constexpr int LDS_DOUBLES = NVT * (HX * HY + NFX + NFY) + NX * NC;
+  static_assert(NFX <= NB && NFY <= NB && NC <= NB, "one pass per job");
+};
+
+// The planes of one fluid (NFL from plane OFF) of a cell and its ghost images.
+template <int NDIM, int NFL, int OFF>
+__device__ __forceinline__ void store_fluid(double* U, const StageArgs& a, int ci, int cj, const double* u) {
+#pragma unroll
+  for (int n = 0; n < NFL; n++) U[(OFF + n) * a.N + (long long)cj * a.ix + ci] = u[n];
+  for_each_image(ci, cj, a.ix, (NDIM == 2) ? a.jx : 1, a.bnd, [&](int xi, int yj, unsigned m) {
+    for (int n = 0; n < NFL; n++)
+      U[(OFF + n) * a.N + (long long)yj * a.ix + xi] = ((m >> (OFF + n)) & 1u) ? -u[n] : u[n];
+  });
+}
+
+template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, bool DIRS, int MODE>
+__global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageArgs a) {
+  using G = SplitGeom<NDIM, NV, TX, TY, DIRS>;
+  constexpr int NVT = G::NVT, NT = G::NT, NB = G::NB, HX = G::HX, HY = G::HY, NC = G::NC;
+  constexpr int NFX = G::NFX, NFY = G::NFY, PV = HX * HY;
+  constexpr int OY = (NDIM == 2) ? 2 : 0;
+  constexpr bool REPLAY = (MODE == STAGE_REPLAY);
+  extern __shared__ double smem[];
+  double* V = smem;
+  double* Fx = V + NVT * PV;
+  double* Fy = Fx + NVT * NFX;
+  double* X = Fy + NVT * NFY;  // Sm (5), um after its rewrites (5), ion_pot, alpha_c, dU0 (5)
+  DevScalars* sc = a.sc;
+  if (!REPLAY && !sc->active) return;
+  const double dt = REPLAY ? a.dtc[0] : sc->dt;
+  const double cmax = REPLAY ? a.dtc[1] : sc->cmax;
+  const int epi = (!REPLAY && a.epi >= 2 && sc->last) ? 1 : a.epi;
+  double c0, c1, dt_sub;
+  stage_coeffs(a.istep, a.t_order, dt, c0, c1, dt_sub);
+  const int ntx = (a.nx + TX - 1) / TX;
+  const int bid = a.xcd_remap ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  const int i0 = (bid % ntx) * TX, j0 = (bid / ntx) * TY;
+  const long long N = a.N;
+  const int ix = a.ix;
+  const int job = __builtin_amdgcn_readfirstlane((int)threadIdx.x / NB), t = (int)threadIdx.x % NB;
+  const int fluid = DIRS ? job >> 1 : job;  // 0 plasma, 1 neutrals
+  const bool cells = !DIRS || (job & 1) == 0;
+  const bool rest = !DIRS || (job & 1) == 1;  // the ring, the y faces
+  const int ti = t % TX, tj = t / TX;
+  const int ci = i0 + ti + 2, cj = (NDIM == 2) ? j0 + tj + 2 : 0;
+  const long long oc = (long long)cj * ix + ci;
+  const bool inside = cells && t < NC && ci < a.ix && cj < a.jx;
+  const bool valid = cells && t < NC && i0 + ti < a.nx && j0 + tj < a.ny;
+
+  // ---- load and convert
+  bool cells_bounded = true;
+  double own[NV], base[NV], other[NV];  // this fluid's cell, its stage base; for the neutrals the plasma's cell
+  auto load = [&](auto fl) {
+    constexpr int FL = decltype(fl)::value, NFL = FL ? 5 : NV, OFF = FL ? NV : 0;
+    auto convert = [&](const double* u0, int hx, int hy, double* v) {
+      double u[NFL], pr, te;
+#pragma unroll
+      for (int n = 0; n < NFL; n++) u[n] = u0[n];
+      for (int k = 0; k < 2; k++)  // set_collisional's, then set_IR's rewrite of E
+        if ((k == 0 && EXT && col_type(a.ph) >= 1) || (k == 1 && IR)) {
+          if constexpr (FL == 0) getpr_mhd(u, pr, te, a.ph);
+          else getpr_hd(u, pr, te, a.ph);
+        }
+      if constexpr (FL == 0) u2v_mhd<NV>(u, v, a.ph);
+      else u2v_hd(u, v, a.ph);
+      cells_bounded = cells_bounded & bounded_cell(v, NFL);
+#pragma unroll
+      for (int n = 0; n < NFL; n++) V[(OFF + n) * PV + hy * HX + hx] = v[n];
+    };
+    if (inside) {
+#pragma unroll
+      for (int n = 0; n < NFL; n++) own[n] = a.Uin[(OFF + n) * N + oc];
+      if (valid) {
+#pragma unroll
+        for (int n = 0; n < NFL; n++) base[n] = a.U0[(OFF + n) * N + oc];
+        if constexpr (FL == 1) {
+#pragma unroll
+          for (int n = 0; n < NV; n++) other[n] = a.Uin[n * N + oc];
+        }
+      }
+    }
+    constexpr int NRX = (NDIM == 2) ? 4 * TX : 0, NR = NRX + 4 * TY;
+    static_assert(NR <= NB, "one pass over the ring");
+    if (rest && t < NR) {
+      const int k = (t < NRX) ? t / TX : (t - NRX) % 4;
+      const int hx = (t < NRX) ? 2 + t % TX : (k < 2 ? k : TX + k);
+      const int hy = (t < NRX) ? (k < 2 ? k : TY + k) : OY + (t - NRX) / 4;
+      const int gi = i0 + hx, gj = (NDIM == 2) ? j0 + hy : 0;
+      if (gi < a.ix && gj < a.jx) {
+        double u[NFL], v[NFL];
+#pragma unroll
+        for (int n = 0; n < NFL; n++) u[n] = a.Uin[(OFF + n) * N + (long long)gj * ix + gi];
+        convert(u, hx, hy, v);
+      }
+    }
+    if (inside) {
+      double v[NFL];
+      convert(own, ti + 2, tj + OY, v);
+      if (MODE != STAGE_PLAIN && a.Vout && valid) store_fluid<NDIM, NFL, OFF>(a.Vout, a, ci, cj, v);
+    }
+  };
+  __shared__ int unbounded[TileBounded<NT>::NW];
+  if (fluid == 0) load(std::integral_constant<int, 0>{});
+  else load(std::integral_constant<int, 1>{});
+  TileBounded<NT>::post(unbounded, cells_bounded);
+  __syncthreads();
+  const bool bounded = TileBounded<NT>::read(unbounded);
+
+  // ---- faces
+  const int xi = t % (TX + 1), xj = t / (TX + 1);
+  const bool xface = t < NFX && i0 + xi <= a.nx && j0 + xj < a.ny;
+  const bool yface = t < NFY && i0 + ti < a.nx && j0 + tj <= a.ny;
+  const double* vx = V + (xj + OY) * HX + xi;
+  const double* vy = V + tj * HX + ti + 2;
+  double acc = a.col, ion_pot = 0.0, S[5], dU0[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  constexpr int PFY = (NDIM == 2) ? NFY : 1;
+  if (fluid == 0) {
+    if (cells && xface) face_flux<0, NV, 0, 1, PV, NFX>(vx, Fx + t, a.ph, cmax, bounded);
+    if (NDIM == 2 && rest && yface) face_flux<0, NV, 1, HX, PV, PFY>(vy, Fy + t, a.ph, cmax, bounded);
+  } else {
+    if (cells && xface) face_flux<1, NV, 0, 1, PV, NFX>(vx + NV * PV, Fx + NV * NFX + t, a.ph, cmax, bounded);
+    if (NDIM == 2 && rest && yface)
+      face_flux<1, NV, 1, HX, PV, PFY>(vy + NV * PV, Fy + NV * NFY + t, a.ph, cmax, bounded);
+    if (valid) {  // sources, as in stage_tile's cell phase
+      if (a.ac) acc = a.ac[oc];
+      if (EXT && col_type(a.ph) >= 1) {
+        acc = set_col_cell(other, own, a.col, a.ph);
+        if (a.ac_out) {
+          a.ac_out[oc] = acc;
+          for_each_image(ci, cj, ix, (NDIM == 2) ? a.jx : 1, a.bnd,
+                         [&](int gx, int gy, unsigned) { a.ac_out[(long long)gy * ix + gx] = acc; });
+        }
+      }
+      double gr = 0.0, gi = 0.0, arb = 0.0;
+      if (IR) {
+        set_ir_cell<NV>(other, own, a.ph, a.irc, gr, gi);
+        if (a.ph.flag_ir_type == 0) arb = a.arb_heat[oc];
+      }
+      const double dtc = (a.t_order == 2) ? dt * 0.5 : dt;
+      Phys phs = a.ph;
+      if (!EXT) phs.pip_imp = 0;
+      double Sm[5];
+      source_pip(other, own, acc, gr, gi, arb, phs, a.irc.heat_fac, S, Sm, ion_pot, dtc, dU0);
+      if (a.ion_pot_out) a.ion_pot_out[oc] = ion_pot;
+#pragma unroll
+      for (int n = 0; n < 5; n++) {
+        X[n * NC + t] = Sm[n];
+        X[(5 + n) * NC + t] = other[n];
+        if (EXT) X[(12 + n) * NC + t] = dU0[n];
+      }
+      X[10 * NC + t] = ion_pot;
+      X[11 * NC + t] = acc;
+    }
+  }
+  __syncthreads();
+
+  // ---- cells
+  RoundOut r = {1.0e300, 0.0, 0.0, 0.0};
+  int nanflag = 0;
+  auto update = [&](auto fl) {
+    constexpr int FL = decltype(fl)::value, NFL = FL ? 5 : NV, OFF = FL ? NV : 0;
+    const bool imp = EXT && a.ph.pip_imp == 1;
+    if constexpr (FL == 0) {
+#pragma unroll
+      for (int n = 0; n < 5; n++) {
+        S[n] = X[n * NC + t];
+        if (EXT) dU0[n] = X[(12 + n) * NC + t];
+        own[n] = X[(5 + n) * NC + t];
+      }
+      ion_pot = X[10 * NC + t];
+      acc = X[11 * NC + t];
+    }
+    const double ax = dt_sub / a.dx, ay = (NDIM == 2) ? dt_sub / a.dy : 0.0;
+    const double* fx = Fx + OFF * NFX + tj * (TX + 1) + ti;
+    const double* fy = Fy + OFF * NFY + t;
+    double un[NFL];
+#pragma unroll
+    for (int n = 0; n < NFL; n++) {
+      double u0 = base[n];
+      if (imp) {
+        if (n < 5) u0 = FL ? u0 - dU0[n] : u0 + dU0[n];
+        if (a.U0out) a.U0out[(OFF + n) * N + oc] = u0;
+      }
+      const double dx = ax * (fx[n * NFX + 1] - fx[n * NFX]);
+      un[n] = (a.istep == 1) ? u0 - dx : c0 * u0 + c1 * own[n] - dx;
+      if (NDIM == 2) un[n] = un[n] - ay * (fy[n * NFY + TX] - fy[n * NFY]);
+      if (n < 5) un[n] = un[n] + S[n] * dt_sub;
+    }
+    if constexpr (FL == 0 && NV == 9) un[8] = un[8] * pexp(-dt_sub / dt * a.ph.safety * a.db_clean);
+    if (epi >= 1) {  // cfl_rewrite and cfl_round of this fluid
+      double pv[8], pr, te;
+      if constexpr (FL == 0) {
+        if (epi >= 2) {
+          if (IR) getpr_mhd(un, pr, te, a.ph);
+          cq2pv_mhd(un, pv, a.ph);
+          if (IR && a.ph.flag_ir_type == 0) getpr_mhd(un, pr, te, a.ph);
+        }
+        if (IR) {
+          double gr, gi;
+          getpr_mhd(un, pr, te, a.ph);
+          ir_rates(un[0], te, a.ph, a.irc, gr, gi);
+          r.gmax = dmax(gr, gi);
+        }
+        r.dtc = cfl_cell_mhd(un, a.gmin_safety, a.ph);
+        r.rhoac = un[0] * acc;
+        if (IR && a.ph.flag_ir_type == 0) {
+          getpr_mhd(un, pr, te, a.ph);
+          r.ratio = fdiv(ion_pot, fdiv(pr, a.ph.gm - 1.0));
+        }
+#pragma unroll
+        for (int n = 0; n < NV; n++) nanflag |= !(un[n] * 0.0 == 0.0);
+      } else {
+        if (epi >= 2) {
+          if (IR) getpr_hd(un, pr, te, a.ph);
+          cq2pv_hd(un, pv, a.ph);
+        }
+        if (IR) getpr_hd(un, pr, te, a.ph);
+        r.dtc = cfl_cell_hd(un, a.gmin_safety, a.ph);
+        r.rhoac = un[0] * acc;
+      }
+    }
+    store_fluid<NDIM, NFL, OFF>(a.Uout, a, ci, cj, un);
+  };
+  if (valid) {
+    if (fluid == 0) update(std::integral_constant<int, 0>{});
+    else update(std::integral_constant<int, 1>{});
+  }
   if (!REPLAY && a.epi >= 1) {
     __syncthreads();
     block_reduce_store<NT, IR>(r, nanflag, valid, a.red[blockIdx.x & (a.nred - 1)].v, smem);

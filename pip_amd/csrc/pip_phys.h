@@ -715,9 +715,8 @@ PIP_HD void source_pip(double* um, double* uh, double ac, double gr, double gi, 
 // ------------------------------------------------------------------- cfl
 // Per-cell terms of cfl_mhd / cfl_hd after their cq2pv rewrites:
 // Scheme_rot.f90:267-278 and :229-241.  Rewrites um/uh.
-template <int NV>
-PIP_HD double cfl_cell(double* um, double* uh, double gmin_safety, const Phys& p) {
-  double pm[8], ph[5];
+PIP_HD double cfl_cell_mhd(double* um, double gmin_safety, const Phys& p) {
+  double pm[8];
   cq2pv_mhd(um, pm, p);
   double de = pm[0], vx = pm[1], vy = pm[2], vz = pm[3], pr = pm[4];
   double bx = pm[5], by = pm[6], bz = pm[7];
@@ -725,12 +724,19 @@ PIP_HD double cfl_cell(double* um, double* uh, double gmin_safety, const Phys& p
   double cs2 = quo(p.gm * pr, dd, rdd);
   double valf2 = quo((bx * bx + by * by) + bz * bz, dd, rdd);
   double vabs = fsqrt((vx * vx + vy * vy) + vz * vz);
-  double dtm = qdiv(gmin_safety, vabs + fsqrt(cs2 + valf2));
+  return qdiv(gmin_safety, vabs + fsqrt(cs2 + valf2));
+}
+PIP_HD double cfl_cell_hd(double* uh, double gmin_safety, const Phys& p) {
+  double ph[5];
   cq2pv_hd(uh, ph, p);
   double cs = fsqrt(qdiv(p.gm * ph[4], ph[0]));
   double vabsn = fsqrt(dmax((ph[1] * ph[1] + ph[2] * ph[2]) + ph[3] * ph[3], kTiny));
-  double dth = qdiv(gmin_safety, vabsn + cs);
-  return dmin(dtm, dth);
+  return qdiv(gmin_safety, vabsn + cs);
+}
+template <int NV>
+PIP_HD double cfl_cell(double* um, double* uh, double gmin_safety, const Phys& p) {
+  const double dtm = cfl_cell_mhd(um, gmin_safety, p);
+  return dmin(dtm, cfl_cell_hd(uh, gmin_safety, p));
 }
 
 }  // namespace PIP_NS

@@ -192,19 +192,55 @@ static int launch_stage_t(pip_ctx* c, const StageArgs& a) {
   return PIP_OK;
 }
 
+template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, bool DIRS, int MODE>
+static int launch_split_t(pip_ctx* c, const StageArgs& a) {
+  using G = SplitGeom<NDIM, NV, TX, TY, DIRS>;
+  constexpr size_t lds = sizeof(double) * (size_t)G::LDS_DOUBLES;
+  static bool attr_done = false;
+  auto kern = k_stage_split<NDIM, NV, IR, EXT, TX, TY, DIRS, MODE>;
+  if (!attr_done) {
+    HIPCHK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    attr_done = true;
+  }
+  const int ntx = (c->nx + TX - 1) / TX, nty = (NDIM == 2) ? (c->ny + TY - 1) / TY : 1;
+  hipLaunchKernelGGL(kern, dim3(ntx * nty), dim3(G::NT), lds, c->stream, a);
+  HIPCHK(hipGetLastError());
+  return PIP_OK;
+}
+
+// Whether the tiles tx x ty of a grid fit one per CU: the split kernel's eight
+// waves per tile (one workgroup per CU) then finish a stage sooner than the
+// one-pass kernel's four, and later once a second round starts.  Stage 1 / 2
+// in us, 16x7 split, 16x15 split, 16x15 one-pass: Orszag-Tang 64^2 (40 and 20
+// tiles) 11.5 / 13.3, 14.6 / 16.4, 16.5 / 18.2; 160^2 (230, 110) 11.9 / 14.8,
+// 14.9 / 16.5, 16.6 / 18.3; 240^2 (525, 240) 22 / 29, 15.2 / 17.0, 16.9 / 18.6;
+// 300^2 (817, 380) 28 / 36, 23.7 / 27.5, 22.1 / 24.8.  1-D, 127-cell split
+// against 255-cell one-pass tiles: 1024 cells 9.7 / 11.2, 11.7 / 13.7.
+constexpr long long kCUs = 256;
+static bool one_round(int nx, int ny, int tx, int ty) {
+  return (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) <= kCUs;
+}
+
 template <int NDIM, int NV, bool IR, bool EXT, int MODE = STAGE_PLAIN>
 static int launch_stage_tile(pip_ctx* c, const StageArgs& a) {
   if constexpr (NDIM == 1) {
+    if (one_round(c->nx, 1, 127, 1)) return launch_split_t<1, NV, IR, EXT, 127, 1, false, MODE>(c, a);
     return launch_stage_t<1, NV, IR, EXT, 255, 1, 256, MODE>(c, a);
   } else {
     // tile shapes (cells) and workgroup sizes; the single-pass shapes keep
     // every face phase within one pass of the workgroup
-    if (c->tx == 16 && c->ty == 15) return launch_stage_t<2, NV, IR, EXT, 16, 15, 256, MODE>(c, a);
+    if (c->tx == 16 && c->ty == 15) {
+      if (one_round(c->nx, c->ny, 16, 15)) return launch_split_t<2, NV, IR, EXT, 16, 15, false, MODE>(c, a);
+      return launch_stage_t<2, NV, IR, EXT, 16, 15, 256, MODE>(c, a);
+    }
     if (c->tx == 32 && c->ty == 7) return launch_stage_t<2, NV, IR, EXT, 32, 7, 256, MODE>(c, a);
     if (c->tx == 32 && c->ty == 15) return launch_stage_t<2, NV, IR, EXT, 32, 15, 512, MODE>(c, a);
     if (c->tx == 64 && c->ty == 7) return launch_stage_t<2, NV, IR, EXT, 64, 7, 512, MODE>(c, a);
     if (c->tx == 32 && c->ty == 8) return launch_stage_t<2, NV, IR, EXT, 32, 8, 256, MODE>(c, a);
-    if (c->tx == 16 && c->ty == 7) return launch_stage_t<2, NV, IR, EXT, 16, 7, 128, MODE>(c, a);
+    if (c->tx == 16 && c->ty == 7) {
+      if (one_round(c->nx, c->ny, 16, 7)) return launch_split_t<2, NV, IR, EXT, 16, 7, true, MODE>(c, a);
+      return launch_stage_t<2, NV, IR, EXT, 16, 7, 128, MODE>(c, a);
+    }
     return fail(PIP_ERR_ARG, "unsupported tile shape");
   }
 }
@@ -444,9 +480,12 @@ int pip_create(const pip_cfg* cfg, pip_ctx** out) {
   // 2.32 ms, 32 of 1024^2 9.35 against 8.63) and within 1 % at 64^2; 1-D tiles
   // share four cells
   c->xcd_remap = cfg->ndim == 2 ? 1 : 0;
-  // by the 16x15 (255-cell) tiles, whatever tile is set: the set count is fixed
+  // grids of at most one 16x7 tile per CU take those (launch_stage_tile's split
+  // kernel), others 16x15
+  if (cfg->ndim == 2 && one_round(c->nx, c->ny, 16, 7)) c->ty = 7;
+  // by the 16x7 (127-cell) tiles, whatever tile is set: the set count is fixed
   // for the context
-  c->nred = red_sets(cfg->ndim == 2 ? (long long)((c->nx + 15) / 16) * ((c->ny + 14) / 15) : (c->nx + 254) / 255);
+  c->nred = red_sets(cfg->ndim == 2 ? (long long)((c->nx + 15) / 16) * ((c->ny + 6) / 7) : (c->nx + 126) / 127);
   hipError_t e;
   size_t bytes = sizeof(double) * (size_t)c->N;
   auto cleanup = [&](const char* what) {

@@ -2,9 +2,11 @@
 against the CPU oracle bit for bit, at the sizes where the choice changes."""
 import numpy as np
 import pytest
+import torch
 
 from oracle.oracle import Oracle
 from pip_amd import problems
+from pip_amd.adjoint import TwoFluidRun
 from pip_amd.solver import PIPSolver
 from tests.util import interior
 
@@ -44,3 +46,63 @@ def test_states_beyond_the_bounded_range(flow, n, power):
     uh *= 2.0 ** power
     um[5:8] *= 2.0 ** (power // 2)
     same_as_oracle(cfg.replace(flag_ir=0, col=cfg.col * 2.0 ** -power), uh, um, None, nsteps=20)
+
+
+def cut(flow, nx, ny, **kw):
+    """An nx x ny corner of a flow's square grid, same cell size."""
+    n = max(nx, ny)
+    cfg, uh, um, _ = getattr(problems, flow)(n)
+    kw.update(nx=nx, ny=ny, xmax=cfg.xmin + nx * cfg.dx, ymax=cfg.ymin + ny * cfg.dy)
+    sl = (slice(None), slice(0, ny + 4), slice(0, nx + 4))
+    return cfg.replace(**kw), uh[sl].copy(), um[sl].copy(), None
+
+
+# default tiles: 16x7 split while they number at most 256, then 16x15 split
+# while those do, then 16x15 one-pass
+SIZES = [(4, 4), (16, 7), (17, 8), (33, 20), (256, 112), (257, 112), (256, 240), (257, 240)]
+
+
+@pytest.mark.parametrize("nx,ny", SIZES)
+@pytest.mark.parametrize("flow,kw", [
+    ("orszag_tang", {}),
+    ("kelvin_helmholtz", {}),
+    ("orszag_tang", dict(t_order=3, flag_bnd=(10, 10, 2, 10))),
+    ("orszag_tang", dict(flag_col=5, col=5.0, flag_pip_imp=1)),
+    ("kelvin_helmholtz", dict(flag_col=4, col=5.0, flag_pip_imp=1)),
+    ("kelvin_helmholtz", dict(flag_divb=0, flag_ir_type=1)),
+], ids=["plain", "ir", "rk3_outflow", "col_imp", "ir_col_imp", "no_psi"])
+def test_split_tiles(nx, ny, flow, kw):
+    """Each path the stage takes by grid size, at the sizes where it changes
+    and at partial tiles, with every option its cell phase splits over."""
+    cfg, uh, um, ac = cut(flow, nx, ny, **kw)
+    if kw.get("flag_divb") == 0:
+        um = um[:8].copy()
+    same_as_oracle(cfg, uh, um, ac, nsteps=3 if nx * ny > 20000 else 8)
+
+
+@pytest.mark.parametrize("nx", [4, 127, 128, 1000, 127 * 256, 127 * 256 + 1])
+@pytest.mark.parametrize("kw", [{}, dict(flag_ir=3), dict(flag_col=2, col=5.0, flag_pip_imp=1, t_order=3)],
+                         ids=["plain", "ir", "col_imp_rk3"])
+def test_split_tiles_1d(nx, kw):
+    cfg, uh, um, ac = problems.brio_wu(nx)
+    same_as_oracle(cfg.replace(**kw), uh, um, ac, nsteps=8)
+
+
+@pytest.mark.parametrize("n", [20, 200])
+@pytest.mark.parametrize("tile", [(16, 7), (16, 15)])
+def test_split_tiles_in_the_adjoints_runs(n, tile):
+    """Recorded and replayed steps (16x7 and 16x15 split, one-pass beyond)
+    end where the plain run does, saved inputs and primitives included."""
+    cfg, uh, um, ac = problems.alfven_damping(n)
+    u0 = torch.from_numpy(np.concatenate([um, uh])).cuda()
+    act = torch.from_numpy(ac).cuda()
+    ends = []
+    for t, keep in ((tile + (1, 0), 2), ((32, 7, 1, 0), 0)):
+        r = TwoFluidRun(cfg, nsteps=6, ckpt_every=2, tile=t, replay_tile=t, keep_segments=keep)
+        a, b = u0.clone().requires_grad_(), act.clone().requires_grad_()
+        out = r.run(a, b)
+        g = torch.autograd.grad((out[:, 2:-2, 2:-2] ** 2).sum(), (a, b))
+        ends.append((out.detach(), *g, r.replay(u0, act)))
+        r.close()
+    for x, y in zip(*ends):
+        assert torch.equal(x, y)
