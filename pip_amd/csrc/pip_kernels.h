@@ -76,6 +76,23 @@ struct DevScalars {
 // an adjoint's recording run).
 enum { STAGE_PLAIN = 0, STAGE_REPLAY = 1, STAGE_SAVE = 2 };
 
+// ---------------------------------------------------------------- step end
+// What the end of a cfl (Scheme_rot.f90:183-213) and of a fused step needs
+// besides the scalars and the reduction slots.  A recorded run also passes
+// hist: at a step's end the next step's {dt, cmax} go to hist[2 hist_k],
+// hist[2 hist_k + 1], as k_record_dt would write them.
+struct FinArgs {
+  DevScalars* sc;
+  RedSlot* red;
+  DevScalars* src;    // the step that ends
+  RedSlot* src_red;
+  int nred;
+  int mode, into_global, flag_ir, flag_ir_type, flag_divb, pip_imp;
+  double safety, dxyz_min, pip_imp_factor;
+  double* hist;
+  int hist_k;
+};
+
 // Boundary description: per side type (1 periodic, 2 mirror, 10 free) and
 // sign masks (bit n set -> variable n flips sign), Boundary_rot.f90:239-320.
 struct StageArgs {
@@ -93,6 +110,8 @@ struct StageArgs {
   DevScalars* sc;
   RedSlot* red;           // reduction slot sets, nred (a power of two) in use
   int nred;
+  int fold;               // split kernel, stage 1: apply the end of the step before (fin) first
+  FinArgs fin;
   int ix, jx, nx, ny;
   long long N;            // plane stride ix*jx
   int istep, t_order, epi;  // epi: 0 none, 1 one cfl round, 2 two rounds + dt reduction
@@ -123,6 +142,112 @@ PIP_HD RedSlot red_slot_init() {
   for (int k = 0; k < RED_N; k++) r.v[k] = 0ull;
   r.v[RED_DT] = as_u64(1.0e300);
   return r;
+}
+
+// The slot sets combined, by one wave: every lane gets the result.
+struct RedVals {
+  double rdt, rhoac, gmax, ratio;
+  int nan;
+};
+__device__ __forceinline__ RedSlot load_slot(const RedSlot* red, int nred, int flag_ir) {
+  const int lane = threadIdx.x & 63;
+  RedSlot rs = red_slot_init();
+  if (lane < nred) {
+    rs.v[RED_DT] = red[lane].v[RED_DT];
+    rs.v[RED_RHOAC] = red[lane].v[RED_RHOAC];
+    rs.v[RED_NAN] = red[lane].v[RED_NAN];
+    if (flag_ir >= 1) {
+      rs.v[RED_GMAX] = red[lane].v[RED_GMAX];
+      rs.v[RED_IONPOT] = red[lane].v[RED_IONPOT];
+    }
+  }
+  return rs;
+}
+__device__ __forceinline__ RedVals combine_slots(RedSlot rs, int nred, int flag_ir) {
+  auto lo = [](unsigned long long a, unsigned long long b) { return a < b ? a : b; };
+  auto hi = [](unsigned long long a, unsigned long long b) { return a > b ? a : b; };
+  for (int off = nred / 2; off > 0; off >>= 1) {  // as the slots' atomics would
+    rs.v[RED_DT] = lo(rs.v[RED_DT], __shfl_xor(rs.v[RED_DT], off, 64));
+    rs.v[RED_RHOAC] = hi(rs.v[RED_RHOAC], __shfl_xor(rs.v[RED_RHOAC], off, 64));
+    if (flag_ir >= 1) {
+      rs.v[RED_GMAX] = hi(rs.v[RED_GMAX], __shfl_xor(rs.v[RED_GMAX], off, 64));
+      rs.v[RED_IONPOT] = hi(rs.v[RED_IONPOT], __shfl_xor(rs.v[RED_IONPOT], off, 64));
+    }
+  }
+  auto first = [](unsigned long long x) {
+    const unsigned l = __builtin_amdgcn_readfirstlane((unsigned)x), h = __builtin_amdgcn_readfirstlane((unsigned)(x >> 32));
+    return as_f64(((unsigned long long)h << 32) | l);
+  };
+  return RedVals{first(rs.v[RED_DT]), first(rs.v[RED_RHOAC]), first(rs.v[RED_GMAX]), first(rs.v[RED_IONPOT]),
+                 __builtin_amdgcn_ballot_w64(rs.v[RED_NAN] != 0ull) != 0ull ? 1 : 0};
+}
+
+// dt of a cfl from its reductions.
+__device__ __forceinline__ double cfl_dt(const RedVals& v, int ion_pot_valid, const FinArgs& f) {
+  double dttemp = dmin(10.0, v.rdt);
+  // cfl_pn_col (Scheme_rot.f90:305-313)
+  if (f.pip_imp == 1) dttemp = dmin(dttemp, f.pip_imp_factor / v.rhoac);
+  else dttemp = dmin(dttemp, dmin(f.safety, 0.3) / v.rhoac);
+  if (f.flag_ir >= 1) {
+    dttemp = dmin(dttemp, dmin(f.safety, 0.1) / dmax(v.gmax, 1.0e-5));
+    if (f.flag_ir_type == 0) {
+      double mx = ion_pot_valid ? v.ratio : 0.0;
+      dttemp = dmin(dttemp, f.safety / dmax(mx, 1.0e-5));
+    }
+  }
+  return dttemp;
+}
+
+// The scalars a step's end reads and writes (DevScalars without its slots).
+struct StepState {
+  double dt, time, cmax, tend, dt_out;
+  long long nt, nmax;
+  int active, last, status, ion_pot_valid;
+};
+__device__ __forceinline__ StepState load_state(const DevScalars* p) {
+  return StepState{p->dt, p->time, p->cmax, p->tend, p->dt_out, p->nt, p->nmax, p->active, p->last, p->status,
+                   p->ion_pot_valid};
+}
+__device__ __forceinline__ void store_state(DevScalars* p, const StepState& s) {
+  p->dt = s.dt;
+  p->time = s.time;
+  p->cmax = s.cmax;
+  p->tend = s.tend;
+  p->dt_out = s.dt_out;
+  p->nt = s.nt;
+  p->nmax = s.nmax;
+  p->active = s.active;
+  p->last = s.last;
+  p->status = s.status;
+  p->ion_pot_valid = s.ion_pot_valid;
+}
+
+__device__ __forceinline__ void record_dt(const StepState& s, double* hist, int k) {
+  hist[2 * k] = s.active ? s.dt : 0.0;
+  hist[2 * k + 1] = s.cmax;
+}
+
+// End of a running fused step: main.f90:58-62 (time += dt, stop_sim), then the
+// next iteration's cfl(dt) and GLM speed and the activity flags.
+__device__ __forceinline__ StepState step_end(StepState s, const RedVals& v, const FinArgs& f) {
+  s.ion_pot_valid = 1;  // source_PIP ran in this step
+  const double dttemp = cfl_dt(v, 1, f);
+  s.dt_out = dttemp;
+  const double dt_used = s.dt;
+  s.time = s.time + dt_used;
+  s.nt = s.nt + 1;
+  int st = 0;
+  if (dt_used <= 1.0e-12) st |= 1;
+  if (v.nan) st |= 2;
+  s.status = st;
+  const bool more = (s.time < s.tend) && (s.nt < s.nmax) && (st == 0);
+  s.active = more ? 1 : 0;
+  if (more) {
+    s.dt = dttemp;
+    if (f.flag_divb >= 1) s.cmax = f.safety * f.dxyz_min / s.dt;
+    s.last = ((s.time + s.dt >= s.tend) || (s.nt + 1 >= s.nmax) || (s.dt <= 1.0e-12)) ? 1 : 0;
+  }
+  return s;
 }
 
 // Store one cell value set (NVT vars) at (ci,cj) and at all its ghost images.
@@ -619,13 +744,15 @@ __global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageA
   double* Fx = V + NVT * PV;
   double* Fy = Fx + NVT * NFX;
   double* X = Fy + NVT * NFY;  // Sm (5), um after its rewrites (5), ion_pot, alpha_c, dU0 (5)
-  DevScalars* sc = a.sc;
-  if (!REPLAY && !sc->active) return;
-  const double dt = REPLAY ? a.dtc[0] : sc->dt;
-  const double cmax = REPLAY ? a.dtc[1] : sc->cmax;
-  const int epi = (!REPLAY && a.epi >= 2 && sc->last) ? 1 : a.epi;
-  double c0, c1, dt_sub;
-  stage_coeffs(a.istep, a.t_order, dt, c0, c1, dt_sub);
+  // the scalars and slots are asked for first and looked at after the cells'
+  // loads have been issued
+  const DevScalars* from = (!REPLAY && a.fold) ? a.fin.src : a.sc;
+  StepState st;
+  RedSlot slot;
+  if (!REPLAY) {
+    st = load_state(from);
+    if (a.fold) slot = load_slot(a.fin.src_red, a.nred, a.fin.flag_ir);
+  }
   const int ntx = (a.nx + TX - 1) / TX;
   const int bid = a.xcd_remap ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
   const int i0 = (bid % ntx) * TX, j0 = (bid / ntx) * TY;
@@ -641,12 +768,70 @@ __global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageA
   const bool inside = cells && t < NC && ci < a.ix && cj < a.jx;
   const bool valid = cells && t < NC && i0 + ti < a.nx && j0 + tj < a.ny;
 
-  // ---- load and convert
-  bool cells_bounded = true;
+  // ---- load
   double own[NV], base[NV], other[NV];  // this fluid's cell, its stage base; for the neutrals the plasma's cell
+  double ring[NV];
+  constexpr int NRX = (NDIM == 2) ? 4 * TX : 0, NR = NRX + 4 * TY;
+  static_assert(NR <= NB, "one pass over the ring");
+  const int rk = (t < NRX) ? t / TX : (t - NRX) % 4;
+  const int rx = (t < NRX) ? 2 + t % TX : (rk < 2 ? rk : TX + rk);
+  const int ry = (t < NRX) ? (rk < 2 ? rk : TY + rk) : OY + (t - NRX) / 4;
+  const int gi = i0 + rx, gj = (NDIM == 2) ? j0 + ry : 0;
+  const bool on_ring = rest && t < NR && gi < a.ix && gj < a.jx;
   auto load = [&](auto fl) {
     constexpr int FL = decltype(fl)::value, NFL = FL ? 5 : NV, OFF = FL ? NV : 0;
-    auto convert = [&](const double* u0, int hx, int hy, double* v) {
+    if (inside) {
+#pragma unroll
+      for (int n = 0; n < NFL; n++) own[n] = a.Uin[(OFF + n) * N + oc];
+    }
+    if (on_ring) {
+#pragma unroll
+      for (int n = 0; n < NFL; n++) ring[n] = a.Uin[(OFF + n) * N + (long long)gj * ix + gi];
+    }
+    if (valid) {
+#pragma unroll
+      for (int n = 0; n < NFL; n++) base[n] = a.U0[(OFF + n) * N + oc];
+      if constexpr (FL == 1) {
+#pragma unroll
+        for (int n = 0; n < NV; n++) other[n] = a.Uin[n * N + oc];
+      }
+    }
+  };
+  if (fluid == 0) load(std::integral_constant<int, 0>{});
+  else load(std::integral_constant<int, 1>{});
+
+  // ---- the step's scalars
+  double dt, cmax;
+  int epi = a.epi;
+  if (REPLAY) {
+    dt = a.dtc[0];
+    cmax = a.dtc[1];
+  } else {
+    if (a.fold) {
+      // every workgroup works out the end of the step before; the first one
+      // writes it where this step's later stages read it, with reset slots
+      if (st.active) st = step_end(st, combine_slots(slot, a.nred, a.fin.flag_ir), a.fin);
+      if (blockIdx.x == 0) {
+        if ((int)threadIdx.x < a.nred) a.red[threadIdx.x] = red_slot_init();
+        if (threadIdx.x == 0) {
+          store_state(a.sc, st);
+          if (a.fin.hist) record_dt(st, a.fin.hist, a.fin.hist_k);
+        }
+      }
+    }
+    if (!st.active) return;
+    dt = st.dt;
+    cmax = st.cmax;
+    if (epi >= 2 && st.last) epi = 1;
+  }
+  double c0, c1, dt_sub;
+  stage_coeffs(a.istep, a.t_order, dt, c0, c1, dt_sub);
+
+  // ---- convert
+  bool cells_bounded = true;
+  auto convert = [&](auto fl) {
+    constexpr int FL = decltype(fl)::value, NFL = FL ? 5 : NV, OFF = FL ? NV : 0;
+    auto one = [&](const double* u0, int hx, int hy, double* v) {
       double u[NFL], pr, te;
 #pragma unroll
       for (int n = 0; n < NFL; n++) u[n] = u0[n];
@@ -661,41 +846,16 @@ __global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageA
 #pragma unroll
       for (int n = 0; n < NFL; n++) V[(OFF + n) * PV + hy * HX + hx] = v[n];
     };
+    double v[NFL];
+    if (on_ring) one(ring, rx, ry, v);
     if (inside) {
-#pragma unroll
-      for (int n = 0; n < NFL; n++) own[n] = a.Uin[(OFF + n) * N + oc];
-      if (valid) {
-#pragma unroll
-        for (int n = 0; n < NFL; n++) base[n] = a.U0[(OFF + n) * N + oc];
-        if constexpr (FL == 1) {
-#pragma unroll
-          for (int n = 0; n < NV; n++) other[n] = a.Uin[n * N + oc];
-        }
-      }
-    }
-    constexpr int NRX = (NDIM == 2) ? 4 * TX : 0, NR = NRX + 4 * TY;
-    static_assert(NR <= NB, "one pass over the ring");
-    if (rest && t < NR) {
-      const int k = (t < NRX) ? t / TX : (t - NRX) % 4;
-      const int hx = (t < NRX) ? 2 + t % TX : (k < 2 ? k : TX + k);
-      const int hy = (t < NRX) ? (k < 2 ? k : TY + k) : OY + (t - NRX) / 4;
-      const int gi = i0 + hx, gj = (NDIM == 2) ? j0 + hy : 0;
-      if (gi < a.ix && gj < a.jx) {
-        double u[NFL], v[NFL];
-#pragma unroll
-        for (int n = 0; n < NFL; n++) u[n] = a.Uin[(OFF + n) * N + (long long)gj * ix + gi];
-        convert(u, hx, hy, v);
-      }
-    }
-    if (inside) {
-      double v[NFL];
-      convert(own, ti + 2, tj + OY, v);
+      one(own, ti + 2, tj + OY, v);
       if (MODE != STAGE_PLAIN && a.Vout && valid) store_fluid<NDIM, NFL, OFF>(a.Vout, a, ci, cj, v);
     }
   };
+  if (fluid == 0) convert(std::integral_constant<int, 0>{});
+  else convert(std::integral_constant<int, 1>{});
   __shared__ int unbounded[TileBounded<NT>::NW];
-  if (fluid == 0) load(std::integral_constant<int, 0>{});
-  else load(std::integral_constant<int, 1>{});
   TileBounded<NT>::post(unbounded, cells_bounded);
   __syncthreads();
   const bool bounded = TileBounded<NT>::read(unbounded);
@@ -1120,91 +1280,37 @@ __global__ void __launch_bounds__(256) k_bnd(double* U, int nvt, int ix, int jx,
   }
 }
 
-// End of cfl: combine the reduction slots into dt (Scheme_rot.f90:183-213).
 // mode 0: pip_cfl (optionally into the global dt); mode 2: the same at the
-// top of a fused loop (also sets active/last); mode 1: end of a fused step
-// (time += dt, stop_sim, next dt and cmax, activity flags).  In mode 1 a
-// recorded run also passes hist: the next step's {dt, cmax} go to
-// hist[2 hist_k], hist[2 hist_k + 1], as k_record_dt would write them.
-struct FinArgs {
-  DevScalars* sc;
-  RedSlot* red;
-  int nred;
-  int mode, into_global, flag_ir, flag_ir_type, flag_divb, pip_imp;
-  double safety, dxyz_min, pip_imp_factor;
-  double* hist;
-  int hist_k;
-};
-
-__device__ __forceinline__ void record_dt(const DevScalars* sc, double* hist, int k) {
-  hist[2 * k] = sc->active ? sc->dt : 0.0;
-  hist[2 * k + 1] = sc->cmax;
-}
-
+// top of a fused loop (also sets active/last); mode 1: end of a fused step.
+// src (mode 1): the scalars and slots of the step that ends, sc / red or the
+// second set of a chunk of folded steps; the result goes to sc.
 __global__ void __launch_bounds__(64) k_finalize(FinArgs f) {
   DevScalars* sc = f.sc;
-  if (f.mode == 1 && !sc->active) {
-    if (f.hist && threadIdx.x == 0) record_dt(sc, f.hist, f.hist_k);
+  if (f.mode == 1) {
+    StepState s = load_state(f.src);
+    if (s.active) s = step_end(s, combine_slots(load_slot(f.src_red, f.nred, f.flag_ir), f.nred, f.flag_ir), f);
+    if ((int)threadIdx.x < f.nred) {
+      f.red[threadIdx.x] = red_slot_init();
+      if (f.src_red != f.red) f.src_red[threadIdx.x] = red_slot_init();
+    }
+    if (threadIdx.x != 0) return;
+    store_state(sc, s);
+    if (f.hist) record_dt(s, f.hist, f.hist_k);
     return;
   }
-  // each of the first lanes takes one slot set and resets it
-  if ((int)threadIdx.x >= f.nred) return;
-  RedSlot rs = f.red[threadIdx.x];
-  f.red[threadIdx.x] = red_slot_init();
-  const int nan = __builtin_amdgcn_ballot_w64(rs.v[RED_NAN] != 0ull) != 0ull;
-  auto lo = [](unsigned long long a, unsigned long long b) { return a < b ? a : b; };
-  auto hi = [](unsigned long long a, unsigned long long b) { return a > b ? a : b; };
-  for (int off = f.nred / 2; off > 0; off >>= 1) {  // as the slots' atomics would
-    rs.v[RED_DT] = lo(rs.v[RED_DT], __shfl_xor(rs.v[RED_DT], off, 64));
-    rs.v[RED_RHOAC] = hi(rs.v[RED_RHOAC], __shfl_xor(rs.v[RED_RHOAC], off, 64));
-    if (f.flag_ir >= 1) {
-      rs.v[RED_GMAX] = hi(rs.v[RED_GMAX], __shfl_xor(rs.v[RED_GMAX], off, 64));
-      rs.v[RED_IONPOT] = hi(rs.v[RED_IONPOT], __shfl_xor(rs.v[RED_IONPOT], off, 64));
-    }
-  }
-  const double rdt = as_f64(rs.v[RED_DT]), rhoac = as_f64(rs.v[RED_RHOAC]);
-  const double gmax = as_f64(rs.v[RED_GMAX]), ratio = as_f64(rs.v[RED_IONPOT]);
+  const RedVals v = combine_slots(load_slot(f.red, f.nred, f.flag_ir), f.nred, f.flag_ir);
+  if ((int)threadIdx.x < f.nred) f.red[threadIdx.x] = red_slot_init();
   if (threadIdx.x != 0) return;
-  if (f.mode == 1) sc->ion_pot_valid = 1;  // source_PIP ran in this step
-  double dttemp = dmin(10.0, rdt);
-  // cfl_pn_col (Scheme_rot.f90:305-313)
-  if (f.pip_imp == 1) dttemp = dmin(dttemp, f.pip_imp_factor / rhoac);
-  else dttemp = dmin(dttemp, dmin(f.safety, 0.3) / rhoac);
-  if (f.flag_ir >= 1) {
-    dttemp = dmin(dttemp, dmin(f.safety, 0.1) / dmax(gmax, 1.0e-5));
-    if (f.flag_ir_type == 0) {
-      double mx = sc->ion_pot_valid ? ratio : 0.0;
-      dttemp = dmin(dttemp, f.safety / dmax(mx, 1.0e-5));
-    }
-  }
+  const double dttemp = cfl_dt(v, sc->ion_pot_valid, f);
   sc->dt_out = dttemp;
-  if (f.mode == 0 || f.mode == 2) {
-    if (f.into_global) sc->dt = dttemp;
-    if (f.flag_divb >= 1) sc->cmax = f.safety * f.dxyz_min / sc->dt;
-    sc->status = nan ? 2 : 0;
-    if (f.mode == 2) {  // top of the time loop: decide whether this step is the last
-      bool go = (sc->time < sc->tend) && (sc->nt < sc->nmax);
-      sc->active = go ? 1 : 0;
-      sc->last = ((sc->time + sc->dt >= sc->tend) || (sc->nt + 1 >= sc->nmax) || (sc->dt <= 1.0e-12)) ? 1 : 0;
-    }
-    return;
-  }
-  // fused step end: main.f90:58-62 then the next iteration's cfl(dt)
-  double dt_used = sc->dt;
-  sc->time = sc->time + dt_used;
-  sc->nt = sc->nt + 1;
-  int st = 0;
-  if (dt_used <= 1.0e-12) st |= 1;
-  if (nan) st |= 2;
-  sc->status = st;
-  bool more = (sc->time < sc->tend) && (sc->nt < sc->nmax) && (st == 0);
-  sc->active = more ? 1 : 0;
-  if (more) {
-    sc->dt = dttemp;
-    if (f.flag_divb >= 1) sc->cmax = f.safety * f.dxyz_min / sc->dt;
+  if (f.into_global) sc->dt = dttemp;
+  if (f.flag_divb >= 1) sc->cmax = f.safety * f.dxyz_min / sc->dt;
+  sc->status = v.nan ? 2 : 0;
+  if (f.mode == 2) {  // top of the time loop: decide whether this step is the last
+    bool go = (sc->time < sc->tend) && (sc->nt < sc->nmax);
+    sc->active = go ? 1 : 0;
     sc->last = ((sc->time + sc->dt >= sc->tend) || (sc->nt + 1 >= sc->nmax) || (sc->dt <= 1.0e-12)) ? 1 : 0;
   }
-  if (f.hist) record_dt(sc, f.hist, f.hist_k);
 }
 
 }  // namespace PIP_NS
@@ -1329,6 +1435,7 @@ __device__ __forceinline__ StageArgs ens_stage_args(const EnsArgs& e, const EnsM
   a.sc = nullptr;
   a.red = nullptr;
   a.nred = 0;
+  a.fold = 0;
   a.ix = M.ix;
   a.jx = 1;
   a.nx = M.nx;
@@ -1749,7 +1856,7 @@ __global__ void k_lock_end(EnsArgs e, DevScalars* scs, const int* members, int c
 // = cmax of step k.
 __global__ void k_record_dt(const DevScalars* sc, double* hist, int k) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  record_dt(sc, hist, k);
+  record_dt(load_state(sc), hist, k);
 }
 // End of a frozen-dt replay of n steps: the scalars a step-by-step run
 // leaves (time and step count advanced, dt / cmax of the last step).

@@ -118,9 +118,12 @@ struct pip_ctx {
 static void build_bnd(pip_ctx* c) { c->bnd = make_bnd(c->cfg.flag_bnd, c->cfg.ndim, c->nv, c->cfg.flag_divb); }
 
 // The scalars of a context and its reduction slots, one device block.
+// The second set is a chunk of folded steps' (odd steps of the chunk).
 struct CtxScalars {
   DevScalars sc;
   RedSlot red[kRedSlots];
+  DevScalars sc1;
+  RedSlot red1[kRedSlots];
 };
 static_assert(sizeof(DevScalars) == 128, "the slots start on a line of their own");
 
@@ -131,7 +134,9 @@ static CtxScalars host_scalars_init() {
   s.sc.red[RED_DT] = as_u64(1.0e300);
   s.sc.nmax = (long long)1 << 62;
   s.sc.active = 1;
+  s.sc1 = s.sc;
   for (auto& r : s.red) r = red_slot_init();
+  for (auto& r : s.red1) r = red_slot_init();
   return s;
 }
 
@@ -155,6 +160,7 @@ static StageArgs stage_args(pip_ctx* c, int istep, const double* Uin, const doub
   a.sc = c->sc;
   a.red = c->red;
   a.nred = c->nred;
+  a.fold = 0;
   a.ix = c->cfg.ix;
   a.jx = c->cfg.jx;
   a.nx = c->nx;
@@ -219,6 +225,13 @@ static int launch_split_t(pip_ctx* c, const StageArgs& a) {
 constexpr long long kCUs = 256;
 static bool one_round(int nx, int ny, int tx, int ty) {
   return (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) <= kCUs;
+}
+
+// The plain context's stages run the split kernel.
+static bool split_stages(const pip_ctx* c) {
+  if (c->arith != PIP_ARITH_EXACT || c->two_pass) return false;
+  if (c->cfg.ndim == 1) return one_round(c->nx, 1, 127, 1);
+  return c->tx == 16 && (c->ty == 7 || c->ty == 15) && one_round(c->nx, c->ny, 16, c->ty);
 }
 
 template <int NDIM, int NV, bool IR, bool EXT, int MODE = STAGE_PLAIN>
@@ -355,11 +368,18 @@ static int launch_round(pip_ctx* c, const RoundArgs& r) {
   return PIP_OK;
 }
 
-// hist / hist_k (mode 1): record the next step's {dt, cmax} at hist_k.
-static int launch_finalize(pip_ctx* c, int mode, int into_global, double* hist = nullptr, int hist_k = 0) {
+// Parity p of a chunk of folded steps: its scalars and slots.
+static DevScalars* scalars(pip_ctx* c, int p) { return p ? &reinterpret_cast<CtxScalars*>(c->sc)->sc1 : c->sc; }
+static RedSlot* slots(pip_ctx* c, int p) { return p ? reinterpret_cast<CtxScalars*>(c->sc)->red1 : c->red; }
+
+// hist / hist_k (mode 1): record the next step's {dt, cmax} at hist_k.  src
+// (mode 1): the parity of the step that ends.
+static FinArgs fin_args(pip_ctx* c, int mode, int into_global, double* hist = nullptr, int hist_k = 0, int src = 0) {
   FinArgs f;
   f.sc = c->sc;
   f.red = c->red;
+  f.src = scalars(c, src);
+  f.src_red = slots(c, src);
   f.nred = c->nred;
   f.hist = hist;
   f.hist_k = hist_k;
@@ -372,7 +392,11 @@ static int launch_finalize(pip_ctx* c, int mode, int into_global, double* hist =
   f.dxyz_min = c->dxyz_min;
   f.pip_imp = c->cfg.flag_pip_imp;
   f.pip_imp_factor = c->cfg.pip_imp_factor;
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, c->stream, f);
+  return f;
+}
+
+static int launch_finalize(pip_ctx* c, int mode, int into_global, double* hist = nullptr, int hist_k = 0, int src = 0) {
+  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, c->stream, fin_args(c, mode, into_global, hist, hist_k, src));
   HIPCHK(hipGetLastError());
   return PIP_OK;
 }
@@ -625,6 +649,35 @@ static int run_stages(pip_ctx* c, int epi_last, double* ion_out) {
   return PIP_OK;
 }
 
+// n steps of the loop; stage(k, s, a) may redirect stage s of step k.  hist:
+// record {dt, cmax} of steps 1..n-1 (step 0's is there).  On the split grids
+// the end of step k - 1 is applied by the first stage of step k (scalars and
+// slots by step parity) instead of by a kernel of its own, whose 4.5 us are as
+// long as half a stage there; on larger grids every workgroup would pay for it
+// again in each round.  A chunk ends on k_finalize either way.
+static int fused_steps(pip_ctx* c, int n, double* hist, const std::function<void(int, int, StageArgs&)>& stage) {
+  const bool fold = split_stages(c);
+  const int T = c->cfg.t_order;
+  for (int k = 0; k < n; k++) {
+    const int p = fold ? (k & 1) : 0;
+    for (int s = 1; s <= T; s++) {
+      const double* Uin = (s == 1) ? c->U : ((s == 2) ? c->U1 : c->U2);
+      double* Uout = (s == T) ? c->U : ((s == 1) ? c->U1 : c->U2);
+      StageArgs a = stage_args(c, s, Uin, c->U, Uout, (s == T) ? 2 : 0, nullptr);
+      a.sc = scalars(c, p);
+      a.red = slots(c, p);
+      if (fold && s == 1 && k > 0) {
+        a.fold = 1;
+        a.fin = fin_args(c, 1, 0, hist, k, p ^ 1);
+      }
+      if (stage) stage(k, s, a);
+      TRY(launch_stage(c, a));
+    }
+    if (!fold || k + 1 == n) TRY(launch_finalize(c, 1, 0, (k + 1 < n) ? hist : nullptr, k + 1, p));
+  }
+  return PIP_OK;
+}
+
 int pip_run_solver(pip_ctx* c) {
   if (!c) return fail(PIP_ERR_ARG, "null context");
   TRY(set_loop(c, 1.0e300, (long long)1 << 62, 1, -1));
@@ -646,11 +699,7 @@ static int loop_top(pip_ctx* c, double tend, long long nmax) {
 }
 
 static int enqueue_fused(pip_ctx* c, int n) {
-  for (int k = 0; k < n; k++) {
-    TRY(run_stages(c, 2, nullptr));
-    TRY(launch_finalize(c, 1, 0));
-  }
-  return PIP_OK;
+  return fused_steps(c, n, nullptr, nullptr);
 }
 
 // The stage-kernel choice a captured chunk depends on.
@@ -999,10 +1048,7 @@ int pip_record_steps(pip_ctx* c, int n, double* hist) {
   if (c->top_pending) TRY(loop_top(c, 1.0e300, (long long)1 << 62));
   // step 0's {dt, cmax} here, step k+1's by the end of step k
   if (n > 0) hipLaunchKernelGGL(k_record_dt, dim3(1), dim3(64), 0, c->stream, c->sc, hist, 0);
-  for (int k = 0; k < n; k++) {
-    TRY(run_stages(c, 2, nullptr));
-    TRY(launch_finalize(c, 1, 0, (k + 1 < n) ? hist : nullptr, k + 1));
-  }
+  TRY(fused_steps(c, n, hist, nullptr));
   HIPCHK(hipGetLastError());
   return PIP_OK;
 }
@@ -1024,18 +1070,14 @@ int pip_record_steps_saved(pip_ctx* c, int n, double* hist, double* Un, double* 
   const size_t S = (size_t)c->N * c->nvt;
   HIPCHK(hipMemcpyAsync(Un, c->U, sizeof(double) * S, hipMemcpyDeviceToDevice, c->stream));
   hipLaunchKernelGGL(k_record_dt, dim3(1), dim3(64), 0, c->stream, c->sc, hist, 0);
-  for (int k = 0; k < n; k++) {
+  TRY(fused_steps(c, n, hist, [&](int k, int s, StageArgs& a) {
     double* un = Un + (size_t)k * S;
     double* u1 = U1 + (size_t)k * S;
-    double* out = (k + 1 < n) ? Un + (size_t)(k + 1) * S : c->U;
-    StageArgs a1 = stage_args(c, 1, un, un, u1, 0, nullptr);
-    StageArgs a2 = stage_args(c, 2, u1, un, out, 2, nullptr);
-    a1.Vout = Vn + (size_t)k * S;
-    a2.Vout = V1 + (size_t)k * S;
-    TRY(launch_stage(c, a1));
-    TRY(launch_stage(c, a2));
-    TRY(launch_finalize(c, 1, 0, (k + 1 < n) ? hist : nullptr, k + 1));
-  }
+    a.Uin = (s == 1) ? un : u1;
+    a.U0 = un;
+    a.Uout = (s == 1) ? u1 : ((k + 1 < n) ? Un + (size_t)(k + 1) * S : c->U);
+    a.Vout = (s == 1 ? Vn : V1) + (size_t)k * S;
+  }));
   HIPCHK(hipGetLastError());
   return PIP_OK;
 }

@@ -106,3 +106,33 @@ def test_split_tiles_in_the_adjoints_runs(n, tile):
         r.close()
     for x, y in zip(*ends):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("flow,n", [("brio_wu", 300), ("orszag_tang", 24), ("kelvin_helmholtz", 20)])
+def test_folded_step_ends(flow, n):
+    """On split grids a step's end runs in the next step's first stage: chunks
+    of odd and even lengths, a run that stops on its end time inside a chunk
+    and goes on, and the procedures in between, against the oracle."""
+    cfg, uh, um, ac = getattr(problems, flow)(n)
+    o = Oracle(cfg, uh, um, ac)
+    s = PIPSolver(cfg, uh, um, ac)
+    for steps in (1, 2, 3, 64, 65, 128):
+        o.run(nsteps=steps)
+        assert s.advance(nsteps=steps)[0] == steps
+        assert (s.scalars()["dt"], s.scalars()["time"]) == (o.scalars()["dt"], o.scalars()["time"])
+    tend = o.scalars()["time"] + 20.5 * o.scalars()["dt"]
+    o.run(tend=tend)
+    s.advance(tend=tend)
+    assert s.scalars()["nt"] == o.scalars()["nt"]
+    o.run(nsteps=5)
+    s.advance(nsteps=5)
+    oh, om = o.state()
+    gh, gm = s.state()
+    assert np.array_equal(interior(gm, cfg), interior(om, cfg)) and np.array_equal(interior(gh, cfg), interior(oh, cfg))
+    assert (s.scalars()["dt"], s.scalars()["time"]) == (o.scalars()["dt"], o.scalars()["time"])
+    # a NaN stops the run at its step's end and is still flagged after it
+    um[6, um.shape[1] // 2, um.shape[2] // 2] = np.nan
+    b = PIPSolver(cfg, uh, um, ac)
+    assert b.advance(nsteps=70)[0] == 1 and b.status() == 2
+    for x in (s, b):
+        x.close()
