@@ -1714,81 +1714,86 @@ __device__ __forceinline__ StageArgs ens_stage_args2(const EnsArgs& e, const Ens
   return a;
 }
 
-// cfl rewrite round over all cells of a 2-D member (ghosts included), as
-// k_round does for the plain path; returns the reduced dt terms.
-template <int NT>
-__device__ __forceinline__ RoundOut ens_cfl_cells2(double* U, const StageArgs& a, double* lds) {
-  RoundOut acc = {1.0e300, 0.0, 0.0, 0.0};
-  int fl = 0;
-  for (long long k = threadIdx.x; k < a.N; k += NT) {
-    double u[14];
-#pragma unroll
-    for (int n = 0; n < 14; n++) u[n] = U[n * a.N + k];
-    const double dtc = cfl_cell<9>(u, u + 9, a.gmin_safety, a.ph);
-    const int i = (int)(k % a.ix), j = (int)(k / a.ix);
-    if (i >= 2 && i < a.ix - 2 && j >= 2 && j < a.jx - 2) acc.dtc = dmin(acc.dtc, dtc);
-    acc.rhoac = dmax(acc.rhoac, dmax(u[0] * a.col, u[9] * a.col));
-#pragma unroll
-    for (int n = 0; n < 14; n++) U[n * a.N + k] = u[n];
+// Start of the 2-D members, three launches over (256 cells, member): the
+// boundary map of the initial state (ghosts from interior sources, k_bnd's
+// composite map) with reset slots; the prologue cfl and the loop-top cfl of
+// every cell (ghosts included, as k_round does; pointwise, so one pass makes
+// both rewrites) reduced into the member's slots; the members' scalars.  One
+// workgroup a member took 1.0 ms for the 68,000 cells of a 256^2 member, these
+// take 0.03.
+__global__ void __launch_bounds__(256) k_lock_bnd2(EnsArgs e, DevScalars* scs) {
+  const int m = blockIdx.y;
+  const EnsMember M = e.mem[m];
+  const long long k = (long long)blockIdx.x * 256 + threadIdx.x, N = (long long)M.ix * M.jx;
+  if (k == 0) {
+    const RedSlot r = red_slot_init();
+    for (int n = 0; n < RED_N; n++) scs[m].red[n] = r.v[n];
   }
-  return wg_reduce<NT>(acc, fl, lds);
+  if (k >= N) return;
+  const int i = (int)(k % M.ix), j = (int)(k / M.ix);
+  const bool gx = (i < 2 || i >= M.ix - 2), gy = (j < 2 || j >= M.jx - 2);
+  if (!gx && !gy) return;
+  bool fx = false, fy = false;
+  const int si = gx ? src_index(i, M.ix, e.bnd.type[0], e.bnd.type[1], fx) : i;
+  const int sj = gy ? src_index(j, M.jx, e.bnd.type[2], e.bnd.type[3], fy) : j;
+  unsigned msk = 0u;
+  if (fx) msk ^= e.bnd.sym[(i < 2) ? 0 : 1];
+  if (fy) msk ^= e.bnd.sym[(j < 2) ? 2 : 3];
+  double* U = e.U + M.off;
+  const long long src = (long long)sj * M.ix + si;
+  for (int n = 0; n < 14; n++) {
+    const double v = U[n * N + src];
+    U[n * N + k] = ((msk >> n) & 1u) ? -v : v;
+  }
 }
 
-// Start of a 2-D member by one workgroup: the boundary map of the initial
-// state (ghosts from interior sources, k_bnd's composite map), the prologue
-// cfl and the loop-top cfl; writes both scalar buffers.
-template <int NT>
-__global__ void __launch_bounds__(NT) k_lock_start2(EnsArgs e, DevScalars* scs) {
-  __shared__ double lds_red[3 * (NT / 64)];
-  const int m = blockIdx.x;
+__global__ void __launch_bounds__(256) k_lock_cfl2(EnsArgs e, DevScalars* scs) {
+  __shared__ double red_lds[4 * 5];
+  const int m = blockIdx.y;
+  const EnsMember M = e.mem[m];
+  const long long k = (long long)blockIdx.x * 256 + threadIdx.x, N = (long long)M.ix * M.jx;
+  if ((long long)blockIdx.x * 256 >= N) return;
+  RoundOut r = {1.0e300, 0.0, 0.0, 0.0};
+  if (k < N) {
+    double* U = e.U + M.off;
+    double u[14];
+#pragma unroll
+    for (int n = 0; n < 14; n++) u[n] = U[n * N + k];
+    cfl_cell<9>(u, u + 9, M.gmin_safety, e.ph);
+    const double dtc = cfl_cell<9>(u, u + 9, M.gmin_safety, e.ph);
+    const int i = (int)(k % M.ix), j = (int)(k / M.ix);
+    if (i >= 2 && i < M.ix - 2 && j >= 2 && j < M.jx - 2) r.dtc = dtc;
+    r.rhoac = dmax(u[0] * M.col, u[9] * M.col);
+#pragma unroll
+    for (int n = 0; n < 14; n++) U[n * N + k] = u[n];
+  }
+  block_reduce_store<256, false>(r, 0, k < N, scs[m].red, red_lds);
+}
+
+__global__ void __launch_bounds__(256) k_lock_init2(EnsArgs e, DevScalars* scs) {
+  const int m = (int)(blockIdx.x * 256 + threadIdx.x);
   if (m >= e.n_members) return;
   const EnsMember M = e.mem[m];
-  const StageArgs a = ens_stage_args2(e, M);
-  double* U = e.U + M.off;
-  for (long long k = threadIdx.x; k < a.N; k += NT) {
-    const int i = (int)(k % a.ix), j = (int)(k / a.ix);
-    const bool gx = (i < 2 || i >= a.ix - 2), gy = (j < 2 || j >= a.jx - 2);
-    if (!gx && !gy) continue;
-    bool fx = false, fy = false;
-    const int si = gx ? src_index(i, a.ix, e.bnd.type[0], e.bnd.type[1], fx) : i;
-    const int sj = gy ? src_index(j, a.jx, e.bnd.type[2], e.bnd.type[3], fy) : j;
-    unsigned msk = 0u;
-    if (fx) msk ^= e.bnd.sym[(i < 2) ? 0 : 1];
-    if (fy) msk ^= e.bnd.sym[(j < 2) ? 2 : 3];
-    const long long src = (long long)sj * a.ix + si;
-    for (int n = 0; n < 14; n++) {
-      const double v = U[n * a.N + src];
-      U[n * a.N + k] = ((msk >> n) & 1u) ? -v : v;
-    }
-  }
-  __syncthreads();
-  ens_cfl_cells2<NT>(U, a, lds_red);
-  __syncthreads();
-  const RoundOut o = ens_cfl_cells2<NT>(U, a, lds_red);
+  const RoundOut o = {as_f64(scs[m].red[RED_DT]), as_f64(scs[m].red[RED_RHOAC]), 0.0, 0.0};
   const double dt = ens_dt(o, e.ph.safety);
-  if (threadIdx.x == 0) {
-    DevScalars sc;
-    sc.dt = dt;
-    sc.time = 0.0;
-    sc.cmax = e.ph.safety * M.dxyz_min / dt;
-    sc.tend = M.tend;
-    sc.dt_out = dt;
-    sc.nt = 0;
-    sc.nmax = M.nmax;
-    sc.status = 0;
-    sc.ion_pot_valid = 0;
-    sc.red[RED_DT] = as_u64(1.0e300);
-    sc.red[RED_RHOAC] = 0ull;
-    sc.red[RED_GMAX] = 0ull;
-    sc.red[RED_IONPOT] = 0ull;
-    sc.red[RED_NAN] = 0ull;
-    const bool go = (0.0 < M.tend) && (0 < M.nmax);
-    sc.active = go ? 1 : 0;
-    sc.last = ((0.0 + dt >= M.tend) || (1 >= M.nmax) || (dt <= 1.0e-12)) ? 1 : 0;
-    scs[m] = sc;
-    scs[e.n_members + m] = sc;
-    if (!go) e.out[m] = EnsOut{0.0, dt, 0, 0, 0};
-  }
+  DevScalars sc;
+  sc.dt = dt;
+  sc.time = 0.0;
+  sc.cmax = e.ph.safety * M.dxyz_min / dt;
+  sc.tend = M.tend;
+  sc.dt_out = dt;
+  sc.nt = 0;
+  sc.nmax = M.nmax;
+  sc.status = 0;
+  sc.ion_pot_valid = 0;
+  const RedSlot r = red_slot_init();
+  for (int n = 0; n < RED_N; n++) sc.red[n] = r.v[n];
+  const bool go = (0.0 < M.tend) && (0 < M.nmax);
+  sc.active = go ? 1 : 0;
+  sc.last = ((0.0 + dt >= M.tend) || (1 >= M.nmax) || (dt <= 1.0e-12)) ? 1 : 0;
+  scs[m] = sc;
+  scs[e.n_members + m] = sc;
+  if (!go) e.out[m] = EnsOut{0.0, dt, 0, 0, 0};
 }
 
 // Stage ISTEP of step k (p = k & 1) for one 16x15 tile of a 2-D member, as

@@ -1496,6 +1496,7 @@ static int ens_kernels_1d(pip_ens* e, EnsKernels* K) {
 }
 
 // The kernels of 2-D members (16x15 tiles).
+constexpr int kGridY = 65535;  // limit of a grid's second dimension
 static int ens_kernels_2d(pip_ens* e, EnsKernels* K) {
   const size_t lds_stage = sizeof(double) * (size_t)TileGeom<2, 9, kEns2TX, kEns2TY>::LDS_DOUBLES;
   static bool attr = false;
@@ -1509,8 +1510,18 @@ static int ens_kernels_2d(pip_ens* e, EnsKernels* K) {
   hipStream_t st = e->stream;
   DevScalars* scs = e->scs;
   const int n = e->n;
+  long long cells = 0;  // of the largest member
+  for (const EnsMember& M : e->hmem) cells = std::max(cells, (long long)M.ix * M.jx);
+  const unsigned nb = (unsigned)((cells + 255) / 256);
   K->start = [=](const EnsArgs& a) {
-    hipLaunchKernelGGL(k_lock_start2<256>, dim3((unsigned)n), dim3(256), 0, st, a, scs);
+    for (int m0 = 0; m0 < n; m0 += kGridY) {  // at most kGridY members a launch
+      EnsArgs b = a;
+      b.mem = a.mem + m0;
+      const unsigned nm = (unsigned)std::min(kGridY, n - m0);
+      hipLaunchKernelGGL(k_lock_bnd2, dim3(nb, nm), dim3(256), 0, st, b, scs + m0);
+      hipLaunchKernelGGL(k_lock_cfl2, dim3(nb, nm), dim3(256), 0, st, b, scs + m0);
+    }
+    hipLaunchKernelGGL(k_lock_init2, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, scs);
   };
   K->stage = [=](const EnsArgs& a, const LockTile* tiles, int istep, int nt, int p, int apply_end) {
     if (istep == 1)
