@@ -356,6 +356,43 @@ __device__ __forceinline__ void block_reduce_store(RoundOut r, int nanflag, bool
   }
 }
 
+// ------------------------------------------------------- start of a stage
+// What a stage needs to know of its step.
+struct StepNow {
+  double dt, cmax;
+  int epi;
+  bool active;
+};
+
+// The scalars (and, with fold, slots) of a stage launch, loaded here and used
+// in begin_step after the caller has issued its cells' loads.
+template <bool REPLAY>
+struct StepLoads {
+  StepState st;
+  RedSlot slot;
+  __device__ __forceinline__ explicit StepLoads(const StageArgs& a) {
+    if (REPLAY) return;
+    st = load_state(a.fold ? a.fin.src : a.sc);
+    if (a.fold) slot = load_slot(a.fin.src_red, a.nred, a.fin.flag_ir);
+  }
+  __device__ __forceinline__ StepNow begin_step(const StageArgs& a) {
+    if (REPLAY) return StepNow{a.dtc[0], a.dtc[1], a.epi, true};
+    if (a.fold) {
+      // every workgroup works out the end of the step before; the first one
+      // writes it where this step's later stages read it, with reset slots
+      if (st.active) st = step_end(st, combine_slots(slot, a.nred, a.fin.flag_ir), a.fin);
+      if (blockIdx.x == 0) {
+        if ((int)threadIdx.x < a.nred) a.red[threadIdx.x] = red_slot_init();
+        if (threadIdx.x == 0) {
+          store_state(a.sc, st);
+          if (a.fin.hist) record_dt(st, a.fin.hist, a.fin.hist_k);
+        }
+      }
+    }
+    return StepNow{st.dt, st.cmax, (a.epi >= 2 && st.last) ? 1 : a.epi, st.active != 0};
+  }
+};
+
 // ------------------------------------------------------------ face fluxes
 // Whether every cell of the tile is bounded (pip_riemann.h): the waves'
 // answers side by side in shared memory, read by all after the barrier that
@@ -452,9 +489,12 @@ struct TileGeom {
 // face phase in a single pass of the workgroup (e.g. 16x15 on 256 threads).
 // Returns whether the calling thread owns a cell; r / nanflag receive the
 // cell's dt terms when epi >= 1.
-template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, int NT, int MODE = STAGE_PLAIN>
-__device__ __forceinline__ bool stage_tile(const StageArgs& a, double dt, double cmax, int epi, int i0,
-                                           int j0, double* smem, RoundOut& r, int& nanflag) {
+// step() is asked for the step's {dt, cmax, epi, active} once the cells' loads
+// have been issued (its own loads then wait beside them); a tile of an inactive
+// run ends there.
+template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, int NT, int MODE = STAGE_PLAIN, class Step>
+__device__ __forceinline__ bool stage_tile(const StageArgs& a, Step step, int i0, int j0, double* smem, RoundOut& r,
+                                           int& nanflag) {
   using G = TileGeom<NDIM, NV, TX, TY>;
   constexpr int NVT = G::NVT;
   constexpr int HX = G::HX;
@@ -465,8 +505,6 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, double dt, double
   constexpr int NF = G::NF;
   double* V = smem;                      // NVT * HY * HX
   double* F = smem + NVT * HY * HX;      // NVT * NF
-  double c0, c1, dt_sub;
-  stage_coeffs(a.istep, a.t_order, dt, c0, c1, dt_sub);
   const int tid = threadIdx.x;
   const long long N = a.N;
   const int ix = a.ix;
@@ -501,6 +539,23 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, double dt, double
 #pragma unroll
     for (int n = 0; n < NVT; n++) raw[n] = a.Uin[n * N + oc];
   }
+  static_assert(NR <= NT, "one pass over the ring");
+  const int rk = (tid < NRX) ? tid / TX : (tid - NRX) % 4;
+  const int rx = (tid < NRX) ? 2 + tid % TX : (rk < 2 ? rk : TX + rk);
+  const int ry = (tid < NRX) ? (rk < 2 ? rk : TY + rk) : OY + (tid - NRX) / 4;
+  const int gi = i0 + rx, gj = (NDIM == 2) ? j0 + ry : 0;
+  const bool on_ring = tid < NR && gi < a.ix && gj < a.jx;
+  double ring[NVT];
+  if (on_ring) {
+#pragma unroll
+    for (int n = 0; n < NVT; n++) ring[n] = a.Uin[n * N + (long long)gj * ix + gi];
+  }
+  const StepNow now = step();
+  if (!now.active) return false;
+  const double dt = now.dt, cmax = now.cmax;
+  const int epi = now.epi;
+  double c0, c1, dt_sub;
+  stage_coeffs(a.istep, a.t_order, dt, c0, c1, dt_sub);
   auto convert = [&](const double* u, int hx, int hy, double* v) {
     double um[NV], uh[5];
 #pragma unroll
@@ -523,24 +578,9 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, double dt, double
 #pragma unroll
     for (int n = 0; n < NVT; n++) V[(n * HY + hy) * HX + hx] = v[n];
   };
-  for (int r = tid; r < NR; r += NT) {
-    int hx, hy;
-    if (r < NRX) {
-      const int k = r / TX;
-      hy = k < 2 ? k : TY + k;
-      hx = 2 + r % TX;
-    } else {
-      const int k = (r - NRX) % 4;
-      hy = OY + (r - NRX) / 4;
-      hx = k < 2 ? k : TX + k;
-    }
-    const int gi = i0 + hx, gj = (NDIM == 2) ? j0 + hy : 0;
-    if (gi < a.ix && gj < a.jx) {
-      double u[NVT], v[NVT];
-#pragma unroll
-      for (int n = 0; n < NVT; n++) u[n] = a.Uin[n * N + (long long)gj * ix + gi];
-      convert(u, hx, hy, v);
-    }
+  if (on_ring) {
+    double v[NVT];
+    convert(ring, rx, ry, v);
   }
   if (inside) {
     double v[NVT];
@@ -676,12 +716,8 @@ __device__ __forceinline__ int xcd_tile(int bid, int nb) {
 template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, int NT, int MODE>
 __global__ void __launch_bounds__(NT, NDIM == 1 ? 3 : 2) k_stage(StageArgs a) {
   extern __shared__ double smem[];
-  DevScalars* sc = a.sc;
   constexpr bool REPLAY = (MODE == STAGE_REPLAY);
-  if (!REPLAY && !sc->active) return;
-  const double dt = REPLAY ? a.dtc[0] : sc->dt;
-  const double cmax = REPLAY ? a.dtc[1] : sc->cmax;
-  const int epi = (!REPLAY && a.epi >= 2 && sc->last) ? 1 : a.epi;
+  StepLoads<REPLAY> loads(a);
   const int ntx = (a.nx + TX - 1) / TX;
   int bid = blockIdx.x;
   if (a.xcd_remap) bid = xcd_tile(bid, gridDim.x);
@@ -689,8 +725,16 @@ __global__ void __launch_bounds__(NT, NDIM == 1 ? 3 : 2) k_stage(StageArgs a) {
   const int j0 = (bid / ntx) * TY;
   RoundOut r;
   int nanflag;
-  bool valid = stage_tile<NDIM, NV, IR, EXT, TX, TY, NT, MODE>(a, dt, cmax, epi, i0, j0, smem, r, nanflag);
-  if (!REPLAY && a.epi >= 1) {
+  bool active = true;
+  const bool valid = stage_tile<NDIM, NV, IR, EXT, TX, TY, NT, MODE>(
+      a,
+      [&] {
+        const StepNow now = loads.begin_step(a);
+        active = now.active;
+        return now;
+      },
+      i0, j0, smem, r, nanflag);
+  if (!REPLAY && a.epi >= 1 && active) {
     __syncthreads();
     block_reduce_store<NT, IR>(r, nanflag, valid, a.red[blockIdx.x & (a.nred - 1)].v, smem);
   }
@@ -744,15 +788,7 @@ __global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageA
   double* Fx = V + NVT * PV;
   double* Fy = Fx + NVT * NFX;
   double* X = Fy + NVT * NFY;  // Sm (5), um after its rewrites (5), ion_pot, alpha_c, dU0 (5)
-  // the scalars and slots are asked for first and looked at after the cells'
-  // loads have been issued
-  const DevScalars* from = (!REPLAY && a.fold) ? a.fin.src : a.sc;
-  StepState st;
-  RedSlot slot;
-  if (!REPLAY) {
-    st = load_state(from);
-    if (a.fold) slot = load_slot(a.fin.src_red, a.nred, a.fin.flag_ir);
-  }
+  StepLoads<REPLAY> loads(a);
   const int ntx = (a.nx + TX - 1) / TX;
   const int bid = a.xcd_remap ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
   const int i0 = (bid % ntx) * TX, j0 = (bid / ntx) * TY;
@@ -800,30 +836,10 @@ __global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageA
   if (fluid == 0) load(std::integral_constant<int, 0>{});
   else load(std::integral_constant<int, 1>{});
 
-  // ---- the step's scalars
-  double dt, cmax;
-  int epi = a.epi;
-  if (REPLAY) {
-    dt = a.dtc[0];
-    cmax = a.dtc[1];
-  } else {
-    if (a.fold) {
-      // every workgroup works out the end of the step before; the first one
-      // writes it where this step's later stages read it, with reset slots
-      if (st.active) st = step_end(st, combine_slots(slot, a.nred, a.fin.flag_ir), a.fin);
-      if (blockIdx.x == 0) {
-        if ((int)threadIdx.x < a.nred) a.red[threadIdx.x] = red_slot_init();
-        if (threadIdx.x == 0) {
-          store_state(a.sc, st);
-          if (a.fin.hist) record_dt(st, a.fin.hist, a.fin.hist_k);
-        }
-      }
-    }
-    if (!st.active) return;
-    dt = st.dt;
-    cmax = st.cmax;
-    if (epi >= 2 && st.last) epi = 1;
-  }
+  const StepNow now = loads.begin_step(a);
+  if (!now.active) return;
+  const double dt = now.dt, cmax = now.cmax;
+  const int epi = now.epi;
   double c0, c1, dt_sub;
   stage_coeffs(a.istep, a.t_order, dt, c0, c1, dt_sub);
 
@@ -1509,7 +1525,7 @@ __global__ void __launch_bounds__(TX) k_ensemble(EnsArgs e) {
       a.Uout = U1;
       a.epi = 0;
       for (int i0 = 0; i0 < M.nx; i0 += TC) {
-        stage_tile<1, 8, false, false, TC, 1, TX>(a, dt, 0.0, 0, i0, 0, smem, r, nanflag);
+        stage_tile<1, 8, false, false, TC, 1, TX>(a, [&] { return StepNow{dt, 0.0, 0, true}; }, i0, 0, smem, r, nanflag);
         __syncthreads();
       }
       __threadfence_block();
@@ -1522,7 +1538,8 @@ __global__ void __launch_bounds__(TX) k_ensemble(EnsArgs e) {
       RoundOut acc = {1.0e300, 0.0, 0.0, 0.0};
       int fl = 0;
       for (int i0 = 0; i0 < M.nx; i0 += TC) {
-        bool v = stage_tile<1, 8, false, false, TC, 1, TX>(a, dt, 0.0, epi, i0, 0, smem, r, nanflag);
+        bool v = stage_tile<1, 8, false, false, TC, 1, TX>(a, [&] { return StepNow{dt, 0.0, epi, true}; }, i0, 0, smem, r,
+                                                          nanflag);
         if (v) {
           acc.dtc = dmin(acc.dtc, r.dtc);
           acc.rhoac = dmax(acc.rhoac, r.rhoac);
@@ -1569,30 +1586,28 @@ struct LockTile {
 };
 
 // The persistent loop's step end for one member: dt of the next step from
-// the reductions, time, step count, status, the active / last flags, and
-// reset slots.  A member that has stopped keeps its state; *stops says
-// whether it stops at this step end.
-__device__ __forceinline__ DevScalars lock_step_end(const DevScalars& sc, const EnsMember& M, double safety,
-                                                   bool* stops) {
-  DevScalars o = sc;
+// the reductions, time, step count, status and the active / last flags.  A
+// member that has stopped keeps its state; *stops says whether it stops at
+// this step end.
+struct LockState {
+  StepState s;
+  unsigned long long dt, rhoac, nan;  // the member's slots
+};
+__device__ __forceinline__ LockState load_lock(const DevScalars* p) {
+  return LockState{load_state(p), p->red[RED_DT], p->red[RED_RHOAC], p->red[RED_NAN]};
+}
+__device__ __forceinline__ StepState lock_step_end(const LockState& l, const EnsMember& M, double safety, bool* stops) {
+  StepState o = l.s;
   *stops = false;
-  if (!sc.active) return o;
-  const RoundOut red = {as_f64(sc.red[RED_DT]), as_f64(sc.red[RED_RHOAC]), 0.0, 0.0};
-  const bool fl = sc.red[RED_NAN] != 0ull;
-  o.red[RED_DT] = as_u64(1.0e300);
-  o.red[RED_RHOAC] = 0ull;
-  o.red[RED_GMAX] = 0ull;
-  o.red[RED_IONPOT] = 0ull;
-  o.red[RED_NAN] = 0ull;
-  const double dt = sc.dt;
+  if (!o.active) return o;
+  const RoundOut red = {as_f64(l.dt), as_f64(l.rhoac), 0.0, 0.0};
+  const double dt = o.dt;
   const double dt_new = ens_dt(red, safety);
-  o.time = sc.time + dt;
-  o.nt = sc.nt + 1;
-  int status = sc.status;
-  if (dt <= 1.0e-12) status |= 1;
-  if (fl) status |= 2;
-  o.status = status;
-  if (o.time < M.tend && o.nt < M.nmax && status == 0) {
+  o.time = o.time + dt;
+  o.nt = o.nt + 1;
+  if (dt <= 1.0e-12) o.status |= 1;
+  if (l.nan != 0ull) o.status |= 2;
+  if (o.time < M.tend && o.nt < M.nmax && o.status == 0) {
     o.dt = dt_new;
     if (M.ny > 0) o.cmax = safety * M.dxyz_min / dt_new;  // GLM speed of 2-D members (psi)
     o.last = ((o.time + dt_new >= M.tend) || (o.nt + 1 >= M.nmax) || (dt_new <= 1.0e-12)) ? 1 : 0;
@@ -1601,6 +1616,13 @@ __device__ __forceinline__ DevScalars lock_step_end(const DevScalars& sc, const 
     *stops = true;
   }
   return o;
+}
+// ... written to p with reset slots.
+__device__ __forceinline__ void store_lock(DevScalars* p, const StepState& s) {
+  store_state(p, s);
+  const RedSlot r = red_slot_init();
+#pragma unroll
+  for (int n = 0; n < RED_N; n++) p->red[n] = r.v[n];
 }
 
 template <int TX>
@@ -1639,6 +1661,42 @@ __global__ void __launch_bounds__(TX) k_lock_start(EnsArgs e, DevScalars* scs) {
   }
 }
 
+// The step's scalars of a member for one of its tiles: stage 1 with apply_end
+// applies the end of the step before (prev) once the tile's loads are issued,
+// and the member's first tile writes it to sc.  stopped(): asked before any
+// load, since the launches after a member's last step find it there.
+template <int ISTEP>
+struct LockStep {
+  const EnsArgs& e;
+  const EnsMember& M;
+  DevScalars* sc;
+  LockState now;
+  bool end, first, active = false;
+  int m;
+  __device__ __forceinline__ LockStep(const EnsArgs& e_, const EnsMember& M_, DevScalars* sc_, const DevScalars* prev,
+                                      int apply_end, int m_, bool first_)
+      : e(e_), M(M_), sc(sc_), end(ISTEP == 1 && apply_end), first(first_), m(m_) {
+    now = load_lock(end ? prev : sc);
+  }
+  __device__ __forceinline__ bool stopped() {
+    if (now.s.active) return false;
+    if (end && first && threadIdx.x == 0) store_lock(sc, now.s);
+    return true;
+  }
+  __device__ __forceinline__ StepNow begin() {
+    if (end) {
+      bool stops;
+      now.s = lock_step_end(now, M, e.ph.safety, &stops);
+      if (first && threadIdx.x == 0) {
+        store_lock(sc, now.s);
+        if (stops) e.out[m] = EnsOut{now.s.time, now.s.dt, now.s.nt, now.s.status, 0};
+      }
+    }
+    active = now.s.active != 0;
+    return StepNow{now.s.dt, now.s.cmax, (ISTEP == 1) ? 0 : (now.s.last ? 1 : 2), active};
+  }
+};
+
 // Stage ISTEP (1 or 2) of step k of the running members, one tile per
 // workgroup; p = k & 1.  Stage 1 with apply_end first applies step k-1's
 // end; stage 2 carries the cfl rounds and reduces into the member's slots.
@@ -1650,23 +1708,6 @@ __global__ void __launch_bounds__(TX, 3) k_lock_stage(EnsArgs e, DevScalars* scs
   const LockTile t = tiles[blockIdx.x];
   const EnsMember M = e.mem[t.m];
   DevScalars* sc = scs + (long long)p * e.n_members + t.m;
-  double dt;
-  int last;
-  if (ISTEP == 1 && apply_end) {
-    bool stops;
-    const DevScalars nw = lock_step_end(scs[(long long)(p ^ 1) * e.n_members + t.m], M, e.ph.safety, &stops);
-    if (t.i0 == 0 && threadIdx.x == 0) {
-      *sc = nw;
-      if (stops) e.out[t.m] = EnsOut{nw.time, nw.dt, nw.nt, nw.status, 0};
-    }
-    if (!nw.active) return;
-    dt = nw.dt;
-    last = nw.last;
-  } else {
-    if (!sc->active) return;
-    dt = sc->dt;
-    last = sc->last;
-  }
   StageArgs a = ens_stage_args(e, M);
   double* U = e.U + M.off;
   double* U1 = e.U1 + M.off;
@@ -1675,11 +1716,12 @@ __global__ void __launch_bounds__(TX, 3) k_lock_stage(EnsArgs e, DevScalars* scs
   a.U0 = U;
   a.Uout = (ISTEP == 1) ? U1 : U;
   a.epi = 0;
-  const int epi = (ISTEP == 1) ? 0 : (last ? 1 : 2);
   RoundOut r;
   int nanflag;
-  const bool valid = stage_tile<1, 8, false, false, TC, 1, TX>(a, dt, 0.0, epi, t.i0, 0, smem, r, nanflag);
-  if (ISTEP == 2) {
+  LockStep<ISTEP> step(e, M, sc, scs + (long long)(p ^ 1) * e.n_members + t.m, apply_end, t.m, t.i0 == 0);
+  if (step.stopped()) return;
+  const bool valid = stage_tile<1, 8, false, false, TC, 1, TX>(a, [&] { return step.begin(); }, t.i0, 0, smem, r, nanflag);
+  if (ISTEP == 2 && step.active) {
     __syncthreads();
     block_reduce_store<TX, false>(r, nanflag, valid, sc->red, smem);
   }
@@ -1807,25 +1849,6 @@ __global__ void __launch_bounds__(kEns2NT, 2) k_lock_stage2(EnsArgs e, DevScalar
   const LockTile t = tiles[xcd_tile(blockIdx.x, gridDim.x)];
   const EnsMember M = e.mem[t.m];
   DevScalars* sc = scs + (long long)p * e.n_members + t.m;
-  double dt, cmax;
-  int last;
-  if (ISTEP == 1 && apply_end) {
-    bool stops;
-    const DevScalars nw = lock_step_end(scs[(long long)(p ^ 1) * e.n_members + t.m], M, e.ph.safety, &stops);
-    if (t.i0 == 0 && t.j0 == 0 && threadIdx.x == 0) {
-      *sc = nw;
-      if (stops) e.out[t.m] = EnsOut{nw.time, nw.dt, nw.nt, nw.status, 0};
-    }
-    if (!nw.active) return;
-    dt = nw.dt;
-    cmax = nw.cmax;
-    last = nw.last;
-  } else {
-    if (!sc->active) return;
-    dt = sc->dt;
-    cmax = sc->cmax;
-    last = sc->last;
-  }
   StageArgs a = ens_stage_args2(e, M);
   double* U = e.U + M.off;
   double* U1 = e.U1 + M.off;
@@ -1834,12 +1857,14 @@ __global__ void __launch_bounds__(kEns2NT, 2) k_lock_stage2(EnsArgs e, DevScalar
   a.U0 = U;
   a.Uout = (ISTEP == 1) ? U1 : U;
   a.epi = 0;
-  const int epi = (ISTEP == 1) ? 0 : (last ? 1 : 2);
   RoundOut r;
   int nanflag;
-  const bool valid = stage_tile<2, 9, false, false, kEns2TX, kEns2TY, kEns2NT>(a, dt, cmax, epi, t.i0, t.j0, smem,
-                                                                               r, nanflag);
-  if (ISTEP == 2) {
+  LockStep<ISTEP> step(e, M, sc, scs + (long long)(p ^ 1) * e.n_members + t.m, apply_end, t.m,
+                       t.i0 == 0 && t.j0 == 0);
+  if (step.stopped()) return;
+  const bool valid = stage_tile<2, 9, false, false, kEns2TX, kEns2TY, kEns2NT>(a, [&] { return step.begin(); }, t.i0,
+                                                                               t.j0, smem, r, nanflag);
+  if (ISTEP == 2 && step.active) {
     __syncthreads();
     block_reduce_store<kEns2NT, false>(r, nanflag, valid, sc->red, smem);
   }
@@ -1853,8 +1878,8 @@ __global__ void k_lock_end(EnsArgs e, DevScalars* scs, const int* members, int c
   if (q >= count) return;
   const int m = members[q];
   bool stops;
-  const DevScalars nw = lock_step_end(scs[(long long)p * e.n_members + m], e.mem[m], e.ph.safety, &stops);
-  scs[(long long)(p ^ 1) * e.n_members + m] = nw;
+  const StepState nw = lock_step_end(load_lock(scs + (long long)p * e.n_members + m), e.mem[m], e.ph.safety, &stops);
+  store_lock(scs + (long long)(p ^ 1) * e.n_members + m, nw);
   if (stops) e.out[m] = EnsOut{nw.time, nw.dt, nw.nt, nw.status, 0};
 }
 // Step bookkeeping for recorded / replayed runs: hist[2k] = dt, hist[2k+1]

@@ -649,14 +649,23 @@ static int run_stages(pip_ctx* c, int epi_last, double* ion_out) {
   return PIP_OK;
 }
 
+// Whether the end of step k - 1 is applied by the first stage of step k
+// (scalars and slots by step parity) instead of by a kernel of its own (4.5
+// us): on the split grids and while the 16x15 tiles are one round of two
+// workgroups per CU.  Every workgroup pays for it again: us per step, folded
+// and not, Orszag-Tang 300^2 41.0 / 42.3, 400^2 58.0 / 58.5, 700^2 137.3 / 136.3,
+// KH + IR 2048^2 1455 / 1419.
+static bool fold_steps(const pip_ctx* c) {
+  if (split_stages(c)) return true;
+  return c->arith == PIP_ARITH_EXACT && !c->two_pass && c->cfg.ndim == 2 &&
+         (long long)((c->nx + 15) / 16) * ((c->ny + 14) / 15) <= 2 * kCUs;
+}
+
 // n steps of the loop; stage(k, s, a) may redirect stage s of step k.  hist:
-// record {dt, cmax} of steps 1..n-1 (step 0's is there).  On the split grids
-// the end of step k - 1 is applied by the first stage of step k (scalars and
-// slots by step parity) instead of by a kernel of its own, whose 4.5 us are as
-// long as half a stage there; on larger grids every workgroup would pay for it
-// again in each round.  A chunk ends on k_finalize either way.
+// record {dt, cmax} of steps 1..n-1 (step 0's is there).  A chunk ends on
+// k_finalize whether or not its steps are folded.
 static int fused_steps(pip_ctx* c, int n, double* hist, const std::function<void(int, int, StageArgs&)>& stage) {
-  const bool fold = split_stages(c);
+  const bool fold = fold_steps(c);
   const int T = c->cfg.t_order;
   for (int k = 0; k < n; k++) {
     const int p = fold ? (k & 1) : 0;
