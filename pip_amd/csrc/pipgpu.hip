@@ -1246,6 +1246,7 @@ struct pip_ens {
   int lgraph_key = 0;               // kernel choice the cached graphs were built for
   int* d_active = nullptr;          // members still running after the chunk
   int* h_active = nullptr;          // pinned copy (written by the graph)
+  hipEvent_t chunk_done[2] = {nullptr, nullptr};
 };
 
 static void ens_drop_graphs(pip_ens* e) {
@@ -1378,13 +1379,14 @@ static int ens_lockstep_run(pip_ens* e, int tc, const EnsKernels& K) {
 // a set of members (members of the set that have stopped return at once:
 // their scalars say inactive), the chunk's closing step end over the set,
 // the count of all members still running and its copy to pinned host
-// memory.  The host replays kGraphBatch chunks between looks at the count.
+// memory.  The host keeps one chunk queued beyond the one whose count it waits
+// for (looking only after every fourth chunk, as long runs do not mind, cost 24
+// members of 96 steps 160 empty ones: 14.8 against 14.2 ms).
 // When half of the set has stopped, the set shrinks to the members still
 // running: their graph is taken from the cache or captured (with its own
 // table), so a rerun of the same ensemble captures nothing.  Same kernels and
 // order as lockstep mode, so the same results.
 constexpr int kLockChunk = 64;  // even: a chunk ends on the parity it started with
-constexpr int kGraphBatch = 4;
 constexpr int kGraphCacheMax = 64;
 
 static int ens_lockgraph_get(pip_ens* e, const EnsArgs& a, int tc, const EnsKernels& K,
@@ -1455,20 +1457,37 @@ static int ens_lockgraph_run(pip_ens* e, int tc, int key, const EnsKernels& K) {
   int listed = e->lgraphs[cur].nm;
   K.start(a);
   HIPCHK(hipGetLastError());
+  // One chunk runs ahead of the count that is looked at, so the device does not
+  // wait for the host, but none beyond the members' step caps.
+  long long cap = 0;
+  for (const EnsMember& M : e->hmem) cap = std::max(cap, M.nmax);
+  long long queued = 0, done = 0;  // chunks
+  auto launch = [&]() -> int {
+    HIPCHK(hipGraphLaunch(e->lgraphs[cur].exec, e->stream));
+    HIPCHK(hipEventRecord(e->chunk_done[queued & 1], e->stream));
+    queued++;
+    return PIP_OK;
+  };
+  TRY(launch());
   for (;;) {
-    for (int b = 0; b < kGraphBatch; b++) HIPCHK(hipGraphLaunch(e->lgraphs[cur].exec, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
-    const int active = *e->h_active;
-    if (active == 0) break;
-    if (2 * active <= listed) {
-      // the chunk's end wrote every listed member's scalars to buffer 0
-      HIPCHK(hipMemcpyAsync(e->h_scs, e->scs, sizeof(DevScalars) * (size_t)e->n, hipMemcpyDeviceToHost,
-                            e->stream));
-      HIPCHK(hipStreamSynchronize(e->stream));
-      for (int m = 0; m < e->n; m++) run[m] = (char)(run[m] && e->h_scs[m].active != 0);
-      TRY(ens_lockgraph_get(e, a, tc, K, run, &cur));
-      listed = e->lgraphs[cur].nm;
+    if (queued - done < 2 && queued < cap / kLockChunk + (cap % kLockChunk ? 1 : 0)) TRY(launch());
+    HIPCHK(hipEventSynchronize(e->chunk_done[done & 1]));
+    done++;
+    // (the chunk ahead may already have lowered it)
+    if (2 * *static_cast<volatile int*>(e->h_active) > listed) {
+      if (queued == done) TRY(launch());
+      continue;
     }
+    HIPCHK(hipStreamSynchronize(e->stream));
+    done = queued;
+    if (*e->h_active == 0) break;
+    // the chunk's end wrote every listed member's scalars to buffer 0
+    HIPCHK(hipMemcpyAsync(e->h_scs, e->scs, sizeof(DevScalars) * (size_t)e->n, hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(hipStreamSynchronize(e->stream));
+    for (int m = 0; m < e->n; m++) run[m] = (char)(run[m] && e->h_scs[m].active != 0);
+    TRY(ens_lockgraph_get(e, a, tc, K, run, &cur));
+    listed = e->lgraphs[cur].nm;
+    TRY(launch());
   }
   return PIP_OK;
 }
@@ -1725,6 +1744,8 @@ int pip_ens_create(const pip_cfg* base, const pip_ens_member* members, int n, pi
   if ((er = hipMalloc(&e->d_active, sizeof(int))) != hipSuccess) return bail("hipMalloc active");
   if ((er = hipHostMalloc((void**)&e->h_active, sizeof(int), hipHostMallocDefault)) != hipSuccess)
     return bail("hipHostMalloc active");
+  for (auto& ev : e->chunk_done)
+    if ((er = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return bail("hipEventCreate");
   if ((er = hipMemcpy(e->mem, e->hmem.data(), sizeof(EnsMember) * n, hipMemcpyHostToDevice)) != hipSuccess) return bail("copy");
   if ((er = hipMemcpy(e->order, order.data(), sizeof(int) * n, hipMemcpyHostToDevice)) != hipSuccess) return bail("copy");
   if ((er = hipMemset(e->U, 0, sizeof(double) * off)) != hipSuccess) return bail("memset");
@@ -1742,6 +1763,8 @@ int pip_ens_destroy(pip_ens* e) {
   ens_drop_graphs(e);
   (void)hipFree(e->d_active);
   if (e->h_active) (void)hipHostFree(e->h_active);
+  for (auto& ev : e->chunk_done)
+    if (ev) (void)hipEventDestroy(ev);
   (void)hipFree(e->U);
   (void)hipFree(e->U1);
   (void)hipFree(e->Uinit);
