@@ -280,7 +280,7 @@ __device__ __forceinline__ RoundOut cfl_round(double* um, double* uh, double ac,
   if (IR && a.ph.flag_ir_type == 0) {
     double pr, te;
     getpr_mhd(um, pr, te, a.ph);  // cfl_pip_ir :321
-    r.ratio = fdiv(ion_pot, fdiv(pr, a.ph.gm - 1.0));
+    r.ratio = qdiv(ion_pot, quo(pr, a.ph.gm - 1.0, a.ph.rgm1));
   }
   return r;
 }
@@ -975,7 +975,7 @@ __global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageA
         r.rhoac = un[0] * acc;
         if (IR && a.ph.flag_ir_type == 0) {
           getpr_mhd(un, pr, te, a.ph);
-          r.ratio = fdiv(ion_pot, fdiv(pr, a.ph.gm - 1.0));
+          r.ratio = qdiv(ion_pot, quo(pr, a.ph.gm - 1.0, a.ph.rgm1));
         }
 #pragma unroll
         for (int n = 0; n < NV; n++) nanflag |= !(un[n] * 0.0 == 0.0);
@@ -1261,7 +1261,7 @@ __global__ void __launch_bounds__(256) k_round(RoundArgs a) {
       if (IR && a.ph.flag_ir_type == 0) {
         double pr, te;
         getpr_mhd(um, pr, te, a.ph);
-        r.ratio = (a.ion_pot && interior) ? a.ion_pot[k] / (pr / (a.ph.gm - 1.0)) : 0.0;
+        r.ratio = (a.ion_pot && interior) ? qdiv(a.ion_pot[k], quo(pr, a.ph.gm - 1.0, a.ph.rgm1)) : 0.0;
       }
       if (interior) {
 #pragma unroll
@@ -1465,7 +1465,7 @@ __device__ __forceinline__ StageArgs ens_stage_args(const EnsArgs& e, const EnsM
   a.dy = 100.0;
   a.db_clean = e.db_clean;
   a.ph = e.ph;
-  a.irc = IRConst{0, 0, 0, 0, 0, 0, 0};
+  a.irc = IRConst{};
   a.bnd = e.bnd;
   return a;
 }

@@ -68,7 +68,11 @@ PIP_HD double sgl(double x) { return (double)(float)x; }  // Fortran default-rea
 // zero, infinite and NaN operands are settled by the fixup alone.  Outside
 // those ends the result is therefore bitwise the IEEE quotient.  Quotients
 // that share a denominator share its refined reciprocal: 4 instructions
-// each instead of 11.  The host build divides.
+// each instead of 11.  Divisors that a run fixes (gm - 1, f_p, rec_fac) bring
+// theirs along.  The stage is bound by its FP64 instructions and their chains:
+// with these forms in set_IR, get_Pr, the sources and the cfl terms as well, a
+// step of 2048^2 Kelvin-Helmholtz with set_IR falls from 1.41 to 1.33 ms, of
+// 1024^2 Orszag-Tang by 1.4 %.  The host build divides.
 #if defined(__HIP_DEVICE_COMPILE__)
 __device__ __forceinline__ double qrcp(double d) {
   double r = __builtin_amdgcn_rcp(d);
@@ -106,16 +110,22 @@ PIP_HD double qsqrt(double x) { return sqrt(x); }
 #endif
 PIP_HD double qdiv(double n, double d) { return quo(n, d, qrcp(d)); }
 
-// fdiv(n, d) and fsqrt(x): the quotients and square roots of the set_IR,
-// get_Pr and cfl terms.  Exact build: the IEEE operations (general sequences,
-// valid over the whole range, as the rates can underflow); relaxed device
-// build: the refined reciprocal times n and qsqrt.
+// k x + y for a power of two k.
+PIP_HD double fma2(double k, double x, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_fma(k, x, y);
+#else
+  return y + k * x;
+#endif
+}
+
+// fdiv(n, d): quotients whose operands can underflow (the ionisation rate of a
+// cold cell).  Exact build: the IEEE operation (general sequence, valid over
+// the whole range); relaxed device build: the refined reciprocal times n.
 #if PIP_RELAXED_DEVICE
 PIP_HD double fdiv(double n, double d) { return n * qrcp(d); }
-PIP_HD double fsqrt(double x) { return qsqrt(x); }
 #else
 PIP_HD double fdiv(double n, double d) { return n / d; }
-PIP_HD double fsqrt(double x) { return sqrt(x); }
 #endif
 
 // ------------------------------------------------------ exp / log / pow
@@ -162,7 +172,7 @@ PIP_HD double plog(double x) {
     m = m * 2.0;
     e = e - 1;
   }
-  double s = fdiv(m - 1.0, m + 1.0);
+  double s = qdiv(m - 1.0, m + 1.0);
   double s2 = s * s;
   double t = 1.0 / 25.0;
   t = t * s2 + 1.0 / 23.0;
@@ -233,8 +243,8 @@ PIP_HD void u2v_mhd(const double* u, double* v, const Phys& p) {
   v[1] = u[1] * roi;
   v[2] = u[2] * roi;
   v[3] = u[3] * roi;
-  double pr = (p.gm - 1.0) * ((u[4] - (0.5 * ((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3])) * roi) -
-                              0.5 * ((u[5] * u[5] + u[6] * u[6]) + u[7] * u[7]));
+  double pr = (p.gm - 1.0) * fma2(-0.5, (u[5] * u[5] + u[6] * u[6]) + u[7] * u[7],
+                                  fma2(-0.5, ((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3]) * roi, u[4]));
   if (pr < p.pr_lim) pr = p.pr_lim;
   v[4] = pr;
   v[5] = u[5];
@@ -251,7 +261,7 @@ PIP_HD void u2v_hd(const double* u, double* v, const Phys& p) {
   v[1] = u[1] * roi;
   v[2] = u[2] * roi;
   v[3] = u[3] * roi;
-  double pr = (p.gm - 1.0) * (u[4] - (0.5 * ((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3])) * roi);
+  double pr = (p.gm - 1.0) * fma2(-0.5, ((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3]) * roi, u[4]);
   if (pr < p.pr_lim) pr = p.pr_lim;
   v[4] = pr;
 }
@@ -263,16 +273,15 @@ PIP_HD void cq2pv_mhd(double* u, double* prim, const Phys& p) {
   const double rde = qrcp(de);
   double vx = quo(u[1], de, rde), vy = quo(u[2], de, rde), vz = quo(u[3], de, rde);
   double bx = u[5], by = u[6], bz = u[7];
-  double pr = (p.gm - 1.0) * ((u[4] - (0.5 * de) * ((vx * vx + vy * vy) + vz * vz)) -
-                              0.5 * ((bx * bx + by * by) + bz * bz));
+  const double v2 = (vx * vx + vy * vy) + vz * vz, b2 = (bx * bx + by * by) + bz * bz;
+  double pr = (p.gm - 1.0) * fma2(-0.5, b2, fma2(-0.5, de * v2, u[4]));
   pr = dmax(pr, p.pr_lim);
   de = dmax(de, p.ro_lim);
   u[0] = de;
   u[1] = vx * de;
   u[2] = vy * de;
   u[3] = vz * de;
-  u[4] = (qdiv(pr, p.gm - 1.0) + (0.5 * de) * ((vx * vx + vy * vy) + vz * vz)) +
-         0.5 * ((bx * bx + by * by) + bz * bz);
+  u[4] = fma2(0.5, b2, fma2(0.5, de * v2, quo(pr, p.gm - 1.0, p.rgm1)));
   prim[0] = de; prim[1] = vx; prim[2] = vy; prim[3] = vz;
   prim[4] = pr; prim[5] = bx; prim[6] = by; prim[7] = bz;
 }
@@ -282,34 +291,36 @@ PIP_HD void cq2pv_hd(double* u, double* prim, const Phys& p) {
   double de = u[0];
   const double rde = qrcp(de);
   double vx = quo(u[1], de, rde), vy = quo(u[2], de, rde), vz = quo(u[3], de, rde);
-  double pr = (p.gm - 1.0) * (u[4] - (0.5 * de) * ((vx * vx + vy * vy) + vz * vz));
+  const double v2 = (vx * vx + vy * vy) + vz * vz;
+  double pr = (p.gm - 1.0) * fma2(-0.5, de * v2, u[4]);
   pr = dmax(pr, p.pr_lim);
   de = dmax(de, p.ro_lim);
   u[0] = de;
   u[1] = vx * de;
   u[2] = vy * de;
   u[3] = vz * de;
-  u[4] = qdiv(pr, p.gm - 1.0) + (0.5 * de) * ((vx * vx + vy * vy) + vz * vz);
+  u[4] = fma2(0.5, de * v2, quo(pr, p.gm - 1.0, p.rgm1));
   prim[0] = de; prim[1] = vx; prim[2] = vy; prim[3] = vz; prim[4] = pr;
 }
 
 // get_Pr_HD (+get_Te_HD), rewrites u[4]: Scheme_rot.f90:83-102
 PIP_HD void getpr_hd(double* u, double& pr, double& te, const Phys& p) {
-  double s = (u[1] * u[1] + u[2] * u[2]) + u[3] * u[3];
-  pr = (p.gm - 1.0) * (u[4] - fdiv(0.5 * s, u[0]));
+  const double r0 = qrcp(u[0]);
+  const double q = quo((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3], u[0], r0);
+  pr = (p.gm - 1.0) * fma2(-0.5, q, u[4]);
   pr = dmax(pr, p.pr_lim);
-  u[4] = fdiv(pr, p.gm - 1.0) + 0.5 * fdiv(s, u[0]);
-  te = p.gm * fdiv(pr, u[0]);
+  u[4] = fma2(0.5, q, quo(pr, p.gm - 1.0, p.rgm1));
+  te = p.gm * quo(pr, u[0], r0);
 }
 
 // get_Pr_MHD (+get_Te_MHD), rewrites u[4]: Scheme_rot.f90:104-128
 PIP_HD void getpr_mhd(double* u, double& pr, double& te, const Phys& p) {
-  double q = ((fdiv((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3], u[0]) + u[5] * u[5]) + u[6] * u[6]) +
-             u[7] * u[7];
-  pr = (p.gm - 1.0) * (u[4] - 0.5 * q);
+  const double r0 = qrcp(u[0]);
+  const double q = ((quo((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3], u[0], r0) + u[5] * u[5]) + u[6] * u[6]) + u[7] * u[7];
+  pr = (p.gm - 1.0) * fma2(-0.5, q, u[4]);
   pr = dmax(pr, p.pr_lim);
-  u[4] = fdiv(pr, p.gm - 1.0) + 0.5 * q;
-  te = (0.5 * p.gm) * fdiv(pr, u[0]);
+  u[4] = fma2(0.5, q, quo(pr, p.gm - 1.0, p.rgm1));
+  te = (0.5 * p.gm) * quo(pr, u[0], r0);
 }
 
 // v2u_1: HLL_rot.f90:1189-1215
@@ -561,6 +572,7 @@ PIP_HD void hlld_flux(const double* v_l, const double* v_r, double gm, double cm
 // Run constants of set_IR case 3 (PIP_rot.f90:185-207); computed once.
 struct IRConst {
   double Te_0, rec_fac, f_p, tfac, sqrt_tfac, k_ion, heat_fac;
+  double a_0, r_rec, r_fp;  // 13.6 / Te_0, 1 / rec_fac, 1 / f_p
 };
 
 PIP_HD IRConst ir_constants(const Phys& p) {
@@ -583,16 +595,21 @@ PIP_HD IRConst ir_constants(const Phys& p) {
     c.heat_fac = 13.6 / p.gm / p.T0 / sgl(8.6173e-5);
   else
     c.heat_fac = 13.6 * p.beta / p.T0 / 2.0 / sgl(8.6173e-5);
+  c.a_0 = 13.6 / c.Te_0;
+  c.r_rec = 1.0 / c.rec_fac;
+  c.r_fp = 1.0 / c.f_p;
   return c;
 }
 
 // Gm_rec, Gm_ion of one cell from rho_p and T_p: PIP_rot.f90:215-217
 PIP_HD void ir_rates(double rho_p, double te_p, const Phys& p, const IRConst& c, double& gr,
                      double& gi) {
-  gr = fdiv(fdiv(rho_p, fsqrt(te_p)) * p.t_ir, c.f_p) * c.sqrt_tfac;
-  double a = fdiv(13.6 / c.Te_0, te_p) * c.tfac;
-  double g = c.k_ion * rho_p * pexp(-a) * ppow(a, 0.39);
-  gi = fdiv(fdiv(fdiv(g, 0.232 + a), c.rec_fac), c.f_p) * p.t_ir;
+  gr = quo(qdiv(rho_p, qsqrt(te_p)) * p.t_ir, c.f_p, c.r_fp) * c.sqrt_tfac;
+  const double a = qdiv(c.a_0, te_p) * c.tfac;
+  const double g = c.k_ion * rho_p * pexp(-a) * ppow(a, 0.39);
+  // cold cells' g underflows, past the range of quo
+  if (g > 1.0e-250) gi = quo(quo(qdiv(g, 0.232 + a), c.rec_fac, c.r_rec), c.f_p, c.r_fp) * p.t_ir;
+  else gi = fdiv(fdiv(fdiv(g, 0.232 + a), c.rec_fac), c.f_p) * p.t_ir;
 }
 
 // set_collisional, one cell, col_type 1..6 (PIP_rot.f90:44-97): get_Te_MHD
@@ -697,9 +714,9 @@ PIP_HD void source_pip(double* um, double* uh, double ac, double gr, double gi, 
     double kin = 0.5 * (gr * de * ((vx * vx + vy * vy) + vz * vz) -
                         gi * nde * ((nvx * nvx + nvy * nvy) + nvz * nvz));
     if (p.flag_ir_type == 2)
-      ds[4] = kin - fdiv(gi * npr, p.gm - 1.0) + fdiv(gr * pr, p.gm - 1.0);
+      ds[4] = kin - quo(gi * npr, p.gm - 1.0, p.rgm1) + quo(gr * pr, p.gm - 1.0, p.rgm1);
     else
-      ds[4] = kin - fdiv(gi * npr, p.gm - 1.0) + fdiv(0.5 * gr * pr, p.gm - 1.0);
+      ds[4] = kin - quo(gi * npr, p.gm - 1.0, p.rgm1) + quo(0.5 * gr * pr, p.gm - 1.0, p.rgm1);
 #pragma unroll
     for (int n = 0; n < 5; n++) {
       Sh[n] = Sh[n] + ds[n];
@@ -723,14 +740,15 @@ PIP_HD double cfl_cell_mhd(double* um, double gmin_safety, const Phys& p) {
   const double dd = dmax(de, kTiny), rdd = qrcp(dd);
   double cs2 = quo(p.gm * pr, dd, rdd);
   double valf2 = quo((bx * bx + by * by) + bz * bz, dd, rdd);
-  double vabs = fsqrt((vx * vx + vy * vy) + vz * vz);
-  return qdiv(gmin_safety, vabs + fsqrt(cs2 + valf2));
+  // 1e-230: qsqrt's range ends at 2^-767; its root is lost in the sound speed
+  double vabs = qsqrt(((vx * vx + vy * vy) + vz * vz) + 1.0e-230);
+  return qdiv(gmin_safety, vabs + qsqrt(cs2 + valf2));
 }
 PIP_HD double cfl_cell_hd(double* uh, double gmin_safety, const Phys& p) {
   double ph[5];
   cq2pv_hd(uh, ph, p);
-  double cs = fsqrt(qdiv(p.gm * ph[4], ph[0]));
-  double vabsn = fsqrt(dmax((ph[1] * ph[1] + ph[2] * ph[2]) + ph[3] * ph[3], kTiny));
+  double cs = qsqrt(qdiv(p.gm * ph[4], ph[0]));
+  double vabsn = qsqrt(dmax((ph[1] * ph[1] + ph[2] * ph[2]) + ph[3] * ph[3], kTiny));
   return qdiv(gmin_safety, vabsn + cs);
 }
 template <int NV>

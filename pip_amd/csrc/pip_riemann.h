@@ -26,15 +26,6 @@
 
 namespace PIP_NS {
 
-// k x + y for a power of two k.
-PIP_HD double fma2(double k, double x, double y) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_fma(k, x, y);
-#else
-  return y + k * x;
-#endif
-}
-
 #if defined(__HIP_DEVICE_COMPILE__)
 #if PIP_RELAXED
 __device__ __forceinline__ double quob(double n, double, double r) { return n * r; }

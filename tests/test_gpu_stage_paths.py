@@ -136,3 +136,14 @@ def test_folded_step_ends(flow, n):
     assert b.advance(nsteps=70)[0] == 1 and b.status() == 2
     for x in (s, b):
         x.close()
+
+
+@pytest.mark.parametrize("n", [33, 300])
+def test_ionisation_rates_that_underflow(n):
+    """Plasma from its own temperature down to where the ionisation rate passes
+    1e-250 (a = 13.6 eV / T near 570) and then zero (near 740)."""
+    cfg, uh, um, ac = problems.kelvin_helmholtz(n)
+    rest = 0.5 * (um[1:4] ** 2).sum(0) / um[0] + 0.5 * (um[5:8] ** 2).sum(0)
+    colder = np.geomspace(1.0, 1.0 / 40.0, um.shape[2])
+    um[4] = (um[4] - rest) * colder + rest
+    same_as_oracle(cfg, uh, um, ac, nsteps=3)
