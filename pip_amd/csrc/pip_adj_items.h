@@ -379,29 +379,38 @@ PIP_HD void adj_gather_fluid(const AdjArgs& a, int dir, int n0, long long o2, lo
   }
 }
 
-// The pointwise part and the transpose of u2v at an interior cell, after the
-// face contributions lv: lam_in = pointwise + u2v^T lv.
-PIP_HD void adj_cell_finish(const AdjArgs& a, long long k, double* lv) {
+// The pointwise part t at an interior cell, and its state u.
+PIP_HD void adj_cell_point(const AdjArgs& a, long long k, double* u, double* t) {
+#pragma unroll
+  for (int n = 0; n < ADJ_NVT; n++) u[n] = a.Uin[n * a.N + k];
+  adj_point_part(a, k, u, u + ADJ_NV, t);
+}
+
+// The transpose of u2v after the face contributions lv:
+// lam_in = pointwise + u2v^T lv, of the fluids asked for.
+template <bool NEUTRAL = true, bool PLASMA = true>
+PIP_HD void adj_cell_store(const AdjArgs& a, long long k, const double* u, const double* t, double* lv) {
   constexpr int NV = ADJ_NV, NVT = ADJ_NVT;
   const long long N = a.N;
-  double u[NVT], lu[NVT], t[NVT];
-#pragma unroll
-  for (int n = 0; n < NVT; n++) u[n] = a.Uin[n * N + k];
-  adj_point_part(a, k, u, u + NV, t);
+  double lu[NVT];
 #pragma unroll
   for (int n = 0; n < NVT; n++) lu[n] = 0.0;
-  u2v_vjp<NV>(u, lv, a.ph, lu);
-  u2v_vjp_hd(u + NV, lv + NV, a.ph, lu + NV);
+  if (PLASMA) u2v_vjp<NV>(u, lv, a.ph, lu);
+  if (NEUTRAL) u2v_vjp_hd(u + NV, lv + NV, a.ph, lu + NV);
 #pragma unroll
-  for (int n = 0; n < NVT; n++) a.lam_in[n * N + k] = t[n] + lu[n];
+  for (int n = PLASMA ? 0 : NV; n < (NEUTRAL ? NVT : NV); n++) a.lam_in[n * N + k] = t[n] + lu[n];
+}
+PIP_HD void adj_cell_finish(const AdjArgs& a, long long k, double* lv) {
+  double u[ADJ_NVT], t[ADJ_NVT];
+  adj_cell_point(a, k, u, t);
+  adj_cell_store(a, k, u, t, lv);
 }
 
 // Sum of the face contributions to the primitives of the cell at (i, j),
-// with the sign map `mask` of a ghost image applied (the plasma's only when
-// NEUTRAL is false).  A face with + cell r
+// with the sign map `mask` of a ghost image applied, of the fluids asked for.  A face with + cell r
 // (stride st) takes V_L from cells r-2, r-1, r and V_R from r-1, r, r+1,
 // with the weights of the recorded minmod branches.
-template <bool NEUTRAL = true>
+template <bool NEUTRAL = true, bool PLASMA = true>
 PIP_HD void adj_gather_at(const AdjArgs& a, int i, int j, unsigned mask, double* lv) {
   constexpr int NV = ADJ_NV;
   const long long o = (long long)j * a.ix + i;
@@ -419,7 +428,8 @@ PIP_HD void adj_gather_at(const AdjArgs& a, int i, int j, unsigned mask, double*
                  v0 = (c >= 2 && c <= hi) ? 1.0 : 0.0, vm = (c - 1 >= 2 && c - 1 <= hi) ? 1.0 : 0.0;
     const CodePair* C = adj_code_pairs(a, dir);
     const CodePair k2 = C[o2], k1 = C[o1], k0 = C[o0], km = C[om];
-    adj_gather_fluid<NV>(a, dir, 0, o2, o1, o0, om, v2, v1, v0, vm, k2.c[0], k1.c[0], k0.c[0], km.c[0], mask, lv);
+    if (PLASMA)
+      adj_gather_fluid<NV>(a, dir, 0, o2, o1, o0, om, v2, v1, v0, vm, k2.c[0], k1.c[0], k0.c[0], km.c[0], mask, lv);
     if (NEUTRAL)
       adj_gather_fluid<5>(a, dir, NV, o2, o1, o0, om, v2, v1, v0, vm, k2.c[1], k1.c[1], k0.c[1], km.c[1], mask, lv);
   }

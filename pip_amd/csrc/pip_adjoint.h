@@ -9,7 +9,9 @@
 //   k_adj_gather        per tile of interior cells: the neutrals' face VJPs
 //                       of every face whose stencil reaches the tile, into
 //                       shared memory, then the gather of both fluids' face
-//                       contributions, the pointwise part and u2v^T.
+//                       contributions, the pointwise part and u2v^T;
+//   k_adj_gather_split  the same on smaller tiles, a wave for each part (grids
+//                       that leave CUs idle).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -121,14 +123,12 @@ __global__ void __launch_bounds__(ADJ_PBS, 1) k_adj_plasma_faces(AdjArgs a) {
 // (20 bits) take 42 KB of shared memory, so three workgroups share a CU at
 // 168 VGPRs.
 constexpr int GT_X = 16, GT_Y = 13;
-constexpr int GT_NFX = (GT_X + 3) * GT_Y;
-constexpr int GT_NFY = GT_X * (GT_Y + 3);
-constexpr int GT_NF = GT_NFX + GT_NFY;
-static_assert(GT_X * GT_Y <= 256 && GT_NF <= 2 * 256, "gather tile");
-
-__host__ __device__ inline int adj_gather_tiles(int nx, int ny) {
-  return ((nx + GT_X - 1) / GT_X) * ((ny + GT_Y - 1) / GT_Y);
-}
+template <int TX, int TY>
+struct GatherTile {
+  static constexpr int NFX = (TX + 3) * TY, NF = NFX + TX * (TY + 3);
+  __host__ __device__ static int tiles(int nx, int ny) { return ((nx + TX - 1) / TX) * ((ny + TY - 1) / TY); }
+};
+static_assert(GT_X * GT_Y <= 256 && GatherTile<GT_X, GT_Y>::NF <= 2 * 256, "gather tile");
 
 // Stage 1 (lam_in then receives the step's result): the blocks past the
 // tiles zero the ghost ring of lam_in, adj_ghost_blocks of them.
@@ -137,17 +137,18 @@ __host__ __device__ inline int adj_ghost_blocks(int ix, int jx) {
 }
 
 // The neutral contributions of one direction at a tile cell from the face
-// table: pairs sp[q * GT_NF + f] of plane NV + q and codes sc[f] at the
+// table: pairs sp[q * NF + f] of plane NV + q and codes sc[f] at the
 // faces f2, f1, f0, fm with + cells c+2, c+1, c, c-1 (faces outside the grid
 // hold zero pairs).  The same products and sums as adj_gather_fluid<5>.
+template <int NF>
 __device__ __forceinline__ void adj_gather_neutral_lds(const FacePair* sp, const unsigned* sc, int f2, int f1,
                                                        int f0, int fm, double* lv) {
   const unsigned k2 = sc[f2], k1 = sc[f1], k0 = sc[f0], km = sc[fm];
 #pragma unroll
   for (int q = 0; q < 5; q++) {
     const int sh = 4 * q;
-    const FacePair p2 = sp[q * GT_NF + f2], p1 = sp[q * GT_NF + f1], p0 = sp[q * GT_NF + f0],
-                   pm = sp[q * GT_NF + fm];
+    const FacePair p2 = sp[q * NF + f2], p1 = sp[q * NF + f1], p0 = sp[q * NF + f0],
+                   pm = sp[q * NF + fm];
     const double acc = (p2.l * wl((k2 >> sh) & 3u, 0)) +
                        (p1.l * wl((k1 >> sh) & 3u, 1) + p1.r * wr((k1 >> (sh + 2)) & 3u, 0)) +
                        (p0.l * wl((k0 >> sh) & 3u, 2) + p0.r * wr((k0 >> (sh + 2)) & 3u, 1)) +
@@ -156,26 +157,76 @@ __device__ __forceinline__ void adj_gather_neutral_lds(const FacePair* sp, const
   }
 }
 
-__global__ void __launch_bounds__(256, 3) k_adj_gather(AdjArgs a) {
-  __shared__ FacePair sp[5 * GT_NF];
-  __shared__ unsigned sc[GT_NF];
-  const int nt = adj_gather_tiles(a.nx, a.ny);
-  if ((int)blockIdx.x >= nt) {
-    const int g = ((int)blockIdx.x - nt) * 256 + (int)threadIdx.x;
-    int i, j;
-    if (g < 4 * a.ix) {
-      const int r = g / a.ix;
-      j = r < 2 ? r : a.jx - 4 + r;
-      i = g % a.ix;
-    } else {
-      const int h = g - 4 * a.ix, c = h % 4;
-      j = 2 + h / 4;
-      i = c < 2 ? c : a.ix - 4 + c;
-      if (j >= a.jx - 2) return;
-    }
-    const long long k = (long long)j * a.ix + i;
+// Block b of the zeroed ghost ring.
+__device__ __forceinline__ void adj_zero_ghosts(const AdjArgs& a, int b) {
+  const int g = b * 256 + (int)threadIdx.x;
+  int i, j;
+  if (g < 4 * a.ix) {
+    const int r = g / a.ix;
+    j = r < 2 ? r : a.jx - 4 + r;
+    i = g % a.ix;
+  } else {
+    const int h = g - 4 * a.ix, c = h % 4;
+    j = 2 + h / 4;
+    i = c < 2 ? c : a.ix - 4 + c;
+    if (j >= a.jx - 2) return;
+  }
+  const long long k = (long long)j * a.ix + i;
 #pragma unroll
-    for (int n = 0; n < ADJ_NVT; n++) a.lam_in[n * a.N + k] = 0.0;
+  for (int n = 0; n < ADJ_NVT; n++) a.lam_in[n * a.N + k] = 0.0;
+}
+
+// Face f of the tile at (i0, j0): the neutrals' VJP into the face table.
+template <int TX, int TY>
+__device__ __forceinline__ void adj_tile_face(const AdjArgs& a, int i0, int j0, int f, FacePair* sp, unsigned* sc) {
+  using G = GatherTile<TX, TY>;
+  int dir, fi, fj;
+  if (f < G::NFX) {
+    dir = 0;
+    fi = i0 - 1 + f % (TX + 3);
+    fj = j0 + f / (TX + 3);
+  } else {
+    const int g = f - G::NFX;
+    dir = 1;
+    fi = i0 + g % TX;
+    fj = j0 - 1 + g / TX;
+  }
+  const bool ok = (dir == 0) ? (fi >= 2 && fi <= a.nx + 2 && fj <= a.ny + 1)
+                             : (fi <= a.nx + 1 && fj >= 2 && fj <= a.ny + 2);
+  double lvl[5], lvr[5];
+  unsigned code = 0u;
+  if (ok) {
+    adj_face_vjp<1>(a, dir, fi, fj, lvl, lvr, [&](unsigned long long c) { code = (unsigned)c; });
+  } else {
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      lvl[q] = 0.0;
+      lvr[q] = 0.0;
+    }
+  }
+  // variable q in the sweep's order is plane adj_perm(NV + q, dir)
+#pragma unroll
+  for (int q = 0; q < 5; q++) sp[(adj_perm(ADJ_NV + q, dir) - ADJ_NV) * G::NF + f] = FacePair{lvl[q], lvr[q]};
+  sc[f] = code;
+}
+
+// The neutral contributions of both directions at the tile's cell (lx, ly).
+template <int TX, int TY>
+__device__ __forceinline__ void adj_tile_neutral(const FacePair* sp, const unsigned* sc, int lx, int ly, double* lv) {
+  using G = GatherTile<TX, TY>;
+  const int bx = ly * (TX + 3) + lx;  // x face with + cell ci-1
+  adj_gather_neutral_lds<G::NF>(sp, sc, bx + 3, bx + 2, bx + 1, bx, lv);
+  const int by = G::NFX + ly * TX + lx;  // y face with + cell cj-1
+  adj_gather_neutral_lds<G::NF>(sp, sc, by + 3 * TX, by + 2 * TX, by + TX, by, lv);
+}
+
+__global__ void __launch_bounds__(256, 3) k_adj_gather(AdjArgs a) {
+  using G = GatherTile<GT_X, GT_Y>;
+  __shared__ FacePair sp[5 * G::NF];
+  __shared__ unsigned sc[G::NF];
+  const int nt = G::tiles(a.nx, a.ny);
+  if ((int)blockIdx.x >= nt) {
+    adj_zero_ghosts(a, (int)blockIdx.x - nt);
     return;
   }
   const int t = xcd_order(blockIdx.x, nt);
@@ -183,36 +234,7 @@ __global__ void __launch_bounds__(256, 3) k_adj_gather(AdjArgs a) {
   const int i0 = (t % ntx) * GT_X + 2, j0 = (t / ntx) * GT_Y + 2;  // first cell of the tile
   // ---- the neutrals' face VJPs of the tile's faces
 #pragma unroll 1
-  for (int f = threadIdx.x; f < GT_NF; f += 256) {
-    int dir, fi, fj;
-    if (f < GT_NFX) {
-      dir = 0;
-      fi = i0 - 1 + f % (GT_X + 3);
-      fj = j0 + f / (GT_X + 3);
-    } else {
-      const int g = f - GT_NFX;
-      dir = 1;
-      fi = i0 + g % GT_X;
-      fj = j0 - 1 + g / GT_X;
-    }
-    const bool ok = (dir == 0) ? (fi >= 2 && fi <= a.nx + 2 && fj <= a.ny + 1)
-                               : (fi <= a.nx + 1 && fj >= 2 && fj <= a.ny + 2);
-    double lvl[5], lvr[5];
-    unsigned code = 0u;
-    if (ok) {
-      adj_face_vjp<1>(a, dir, fi, fj, lvl, lvr, [&](unsigned long long c) { code = (unsigned)c; });
-    } else {
-#pragma unroll
-      for (int q = 0; q < 5; q++) {
-        lvl[q] = 0.0;
-        lvr[q] = 0.0;
-      }
-    }
-    // variable q in the sweep's order is plane adj_perm(NV + q, dir)
-#pragma unroll
-    for (int q = 0; q < 5; q++) sp[(adj_perm(ADJ_NV + q, dir) - ADJ_NV) * GT_NF + f] = FacePair{lvl[q], lvr[q]};
-    sc[f] = code;
-  }
+  for (int f = threadIdx.x; f < G::NF; f += 256) adj_tile_face<GT_X, GT_Y>(a, i0, j0, f, sp, sc);
   __syncthreads();
   // ---- the gather at the tile's cells
   if ((int)threadIdx.x >= GT_X * GT_Y) return;
@@ -222,14 +244,7 @@ __global__ void __launch_bounds__(256, 3) k_adj_gather(AdjArgs a) {
   double lv[ADJ_NVT];
 #pragma unroll
   for (int n = 0; n < ADJ_NVT; n++) lv[n] = 0.0;
-  {
-    const int b = ly * (GT_X + 3) + lx;  // x face with + cell ci-1
-    adj_gather_neutral_lds(sp, sc, b + 3, b + 2, b + 1, b, lv);
-  }
-  {
-    const int b = GT_NFX + ly * GT_X + lx;  // y face with + cell cj-1
-    adj_gather_neutral_lds(sp, sc, b + 3 * GT_X, b + 2 * GT_X, b + GT_X, b, lv);
-  }
+  adj_tile_neutral<GT_X, GT_Y>(sp, sc, lx, ly, lv);
   // The sums are formed here: left to the compiler, the shared-memory loads
   // and their weights stay live into the plasma gather (~260 registers).
 #pragma unroll
@@ -240,6 +255,69 @@ __global__ void __launch_bounds__(256, 3) k_adj_gather(AdjArgs a) {
   for_each_image(ci, cj, a.ix, a.jx, a.bnd,
                  [&](int xi, int yj, unsigned m) { adj_gather_at(a, xi, yj, m, lv); });
   adj_cell_finish(a, (long long)cj * a.ix + ci, lv);
+}
+
+// The gather of a grid that leaves CUs idle: what one thread of k_adj_gather
+// does in turn -- two face VJPs, the plasma's gather at the cell and its
+// images, the pointwise part, the neutrals' gather -- is a chain of 30 us
+// there.  Tiles of 8 x 8 cells with a wave for each part: wave 0 the plasma's
+// gather, wave 1 the pointwise part and, after the barrier, the neutrals'
+// gather, waves 2 to 4 one face VJP a thread (176 faces).  The transposes of
+// u2v do not mix the fluids, so wave 0 ends with the plasma's planes, wave 1
+// with the neutrals'.
+constexpr int GS = 8, GS_NT = 320;
+__global__ void __launch_bounds__(GS_NT, 1) k_adj_gather_split(AdjArgs a) {
+  using G = GatherTile<GS, GS>;
+  static_assert(GS * GS == 64 && G::NF <= GS_NT - 128, "two waves of cells, the others of faces");
+  __shared__ FacePair sp[5 * G::NF];
+  __shared__ unsigned sc[G::NF];
+  __shared__ double st[ADJ_NV * 64];  // the pointwise part of the plasma's planes
+  const int nt = G::tiles(a.nx, a.ny);
+  if ((int)blockIdx.x >= nt) {
+    if (threadIdx.x < 256) adj_zero_ghosts(a, (int)blockIdx.x - nt);
+    return;
+  }
+  const int t = xcd_order(blockIdx.x, nt);
+  const int ntx = (a.nx + GS - 1) / GS;
+  const int i0 = (t % ntx) * GS + 2, j0 = (t / ntx) * GS + 2;
+  const int wave = (int)threadIdx.x / 64, c = (int)threadIdx.x % 64;
+  const int lx = c % GS, ly = c / GS;
+  const int ci = i0 + lx, cj = j0 + ly;
+  const long long k = (long long)cj * a.ix + ci;
+  const bool cell = ci <= a.nx + 1 && cj <= a.ny + 1;
+  double lv[ADJ_NVT], u[ADJ_NVT], tp[ADJ_NVT];
+#pragma unroll
+  for (int n = 0; n < ADJ_NVT; n++) lv[n] = 0.0;
+  if (wave == 0) {
+    if (cell) {
+#pragma unroll
+      for (int n = 0; n < ADJ_NV; n++) u[n] = a.Uin[n * a.N + k];
+      adj_gather_at<false>(a, ci, cj, 0u, lv);
+      for_each_image(ci, cj, a.ix, a.jx, a.bnd,
+                     [&](int xi, int yj, unsigned m) { adj_gather_at<false>(a, xi, yj, m, lv); });
+    }
+  } else if (wave == 1) {
+    if (cell) {
+      adj_cell_point(a, k, u, tp);
+#pragma unroll
+      for (int n = 0; n < ADJ_NV; n++) st[n * 64 + c] = tp[n];
+    }
+  } else {
+    const int f = (int)threadIdx.x - 128;
+    if (f < G::NF) adj_tile_face<GS, GS>(a, i0, j0, f, sp, sc);
+  }
+  __syncthreads();
+  if (wave >= 2 || !cell) return;
+  if (wave == 0) {
+#pragma unroll
+    for (int n = 0; n < ADJ_NV; n++) tp[n] = st[n * 64 + c];
+    adj_cell_store<false, true>(a, k, u, tp, lv);
+  } else {
+    adj_tile_neutral<GS, GS>(sp, sc, lx, ly, lv);
+    for_each_image(ci, cj, a.ix, a.jx, a.bnd,
+                   [&](int xi, int yj, unsigned m) { adj_gather_at<true, false>(a, xi, yj, m, lv); });
+    adj_cell_store<true, false>(a, k, u, tp, lv);
+  }
 }
 
 __global__ void __launch_bounds__(256) k_adj_fold_seed(double* lam, int nvt, int ix, int jx, long long N,

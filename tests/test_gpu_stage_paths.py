@@ -1,12 +1,16 @@
 """The paths the stage kernels and the step loop choose by size and state,
 against the CPU oracle bit for bit, at the sizes where the choice changes."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle.oracle import Oracle
 from pip_amd import problems
+from pip_amd._lib import check, lib
 from pip_amd.adjoint import TwoFluidRun
+from pip_amd.config import PIPConfig
 from pip_amd.solver import PIPSolver
 from tests.util import interior
 
@@ -147,3 +151,42 @@ def test_ionisation_rates_that_underflow(n):
     colder = np.geomspace(1.0, 1.0 / 40.0, um.shape[2])
     um[4] = (um[4] - rest) * colder + rest
     same_as_oracle(cfg, uh, um, ac, nsteps=3)
+
+
+@pytest.mark.parametrize("nx,ny", [(4, 4), (8, 8), (9, 17), (65, 48), (128, 128), (129, 128), (40, 523)])
+@pytest.mark.parametrize("bnd", [(1, 1, 1, 1), (2, 2, 3, 2)], ids=["periodic", "mirror"])
+def test_adjoint_gathers(nx, ny, bnd):
+    """One adjoint step on 8 x 8 gather tiles (up to 256 of them) and on
+    16 x 13 ones against the host build of the work items, at the bar of
+    test_adjoint_step_equals_host_work_items."""
+    from tests.test_adjoint_cpu import L as host, _smooth_state
+    cfg = PIPConfig(ndim=2, nx=nx, ny=ny, xmin=0.0, xmax=1.0, ymin=0.0, ymax=ny / nx, flag_divb=1, ac_field=True,
+                    flag_bnd=bnd, col=30.0)
+    o = Oracle(cfg, *_smooth_state(cfg, 5), prologue=False)
+    o.pipbnd()
+    uh, um = o.state()
+    ac = _smooth_state(cfg, 5)[2]
+    dt = 0.05 * min(cfg.dx, cfg.dy)
+    cmax = cfg.safety * min(cfg.dx, cfg.dy) / dt
+    o.set_scalars(dt, cmax)
+    U1 = np.ascontiguousarray(o.run_solver_stage1())
+    U = np.ascontiguousarray(np.concatenate([um, uh]))
+    W = np.random.default_rng(17).normal(size=U.shape)
+    lam_h, lam_ac_h = W.copy(), np.zeros((cfg.jx, cfg.ix))
+    P, I = ctypes.POINTER(ctypes.c_double), ctypes.c_int
+    host.hc_adj_step.argtypes = [I, I, P, ctypes.POINTER(I), P, P, P, P, P]
+    prm = np.array([cfg.gm, cfg.ro_lim, cfg.pr_lim, cfg.dx, cfg.dy, cfg.col, cfg.safety, cfg.db_clean, dt, cmax])
+    host.hc_adj_step(cfg.ix, cfg.jx, prm.ctypes.data_as(P), (I * 4)(*bnd),
+                     *(x.ctypes.data_as(P) for x in (U, U1, np.ascontiguousarray(ac), lam_h, lam_ac_h)))
+    s = PIPSolver(cfg, uh, um, ac, prologue=False)
+    Ud, U1d, lam = (torch.tensor(x, device="cuda:0") for x in (U, U1, W))
+    dtc = torch.tensor([dt, cmax], dtype=torch.float64, device="cuda:0")
+    lam_ac = torch.zeros((cfg.jx, cfg.ix), dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    check(lib().pip_adj_seed(s.h, lam.data_ptr()))
+    check(lib().pip_adj_step(s.h, Ud.data_ptr(), U1d.data_ptr(), None, None, dtc.data_ptr(), lam.data_ptr(),
+                             lam_ac.data_ptr()))
+    s.sync()
+    for g, h in ((lam, lam_h), (lam_ac, lam_ac_h)):
+        assert np.abs(g.cpu().numpy() - h).max() <= 1e-13 * np.abs(h).max()
+    s.close()
