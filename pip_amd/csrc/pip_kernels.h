@@ -492,7 +492,8 @@ struct TileGeom {
 // step() is asked for the step's {dt, cmax, epi, active} once the cells' loads
 // have been issued (its own loads then wait beside them); a tile of an inactive
 // run ends there.
-template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, int NT, int MODE = STAGE_PLAIN, class Step>
+template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, int NT, int MODE = STAGE_PLAIN, bool BF = NDIM == 2,
+          class Step>
 __device__ __forceinline__ bool stage_tile(const StageArgs& a, Step step, int i0, int j0, double* smem, RoundOut& r,
                                            int& nanflag) {
   using G = TileGeom<NDIM, NV, TX, TY>;
@@ -523,8 +524,8 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, Step step, int i0
   const long long oc = (long long)cj * ix + ci;
   // 1-D tiles take the general fluxes: at the 168 registers of three
   // workgroups per CU the bounded ones spill, and few tiles are bound by their
-  // latency (1024 cells: 5.63 against 5.44 ms for 256 steps)
-  constexpr bool BF = NDIM == 2;
+  // latency (1024 cells: 5.63 against 5.44 ms for 256 steps),
+  // unless they ask for them (k_lock_stage).
   __shared__ int unbounded[TileBounded<NT>::NW];
   bool cells_bounded = true;
   constexpr int NRX = (NDIM == 2) ? 4 * TX : 0;  // ring cells above and below
@@ -1700,7 +1701,8 @@ struct LockStep {
 // Stage ISTEP (1 or 2) of step k of the running members, one tile per
 // workgroup; p = k & 1.  Stage 1 with apply_end first applies step k-1's
 // end; stage 2 carries the cfl rounds and reduces into the member's slots.
-template <int TX, int ISTEP>
+// BF: tiles of bounded cells take the bounded fluxes.
+template <int TX, int ISTEP, bool BF>
 __global__ void __launch_bounds__(TX, 3) k_lock_stage(EnsArgs e, DevScalars* scs, const LockTile* tiles, int p,
                                                    int apply_end) {
   extern __shared__ double smem[];
@@ -1720,7 +1722,7 @@ __global__ void __launch_bounds__(TX, 3) k_lock_stage(EnsArgs e, DevScalars* scs
   int nanflag;
   LockStep<ISTEP> step(e, M, sc, scs + (long long)(p ^ 1) * e.n_members + t.m, apply_end, t.m, t.i0 == 0);
   if (step.stopped()) return;
-  const bool valid = stage_tile<1, 8, false, false, TC, 1, TX>(a, [&] { return step.begin(); }, t.i0, 0, smem, r, nanflag);
+  const bool valid = stage_tile<1, 8, false, false, TC, 1, TX, STAGE_PLAIN, BF>(a, [&] { return step.begin(); }, t.i0, 0, smem, r, nanflag);
   if (ISTEP == 2 && step.active) {
     __syncthreads();
     block_reduce_store<TX, false>(r, nanflag, valid, sc->red, smem);

@@ -1510,10 +1510,9 @@ static int ens_kernels_1d(pip_ens* e, EnsKernels* K) {
   if (!attr) {
     HIPCHK(hipFuncSetAttribute((const void*)k_lock_start<TX>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds_start));
-    HIPCHK(hipFuncSetAttribute((const void*)k_lock_stage<TX, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)lds_stage));
-    HIPCHK(hipFuncSetAttribute((const void*)k_lock_stage<TX, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)lds_stage));
+    for (const void* f : {(const void*)k_lock_stage<TX, 1, false>, (const void*)k_lock_stage<TX, 2, false>,
+                          (const void*)k_lock_stage<TX, 1, true>, (const void*)k_lock_stage<TX, 2, true>})
+      HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_stage));
     attr = true;
   }
   hipStream_t st = e->stream;
@@ -1523,10 +1522,14 @@ static int ens_kernels_1d(pip_ens* e, EnsKernels* K) {
     hipLaunchKernelGGL(k_lock_start<TX>, dim3((unsigned)n), dim3(TX), lds_start, st, a, scs);
   };
   K->stage = [=](const EnsArgs& a, const LockTile* tiles, int istep, int nt, int p, int apply_end) {
-    if (istep == 1)
-      hipLaunchKernelGGL((k_lock_stage<TX, 1>), dim3((unsigned)nt), dim3(TX), lds_stage, st, a, scs, tiles, p, apply_end);
-    else
-      hipLaunchKernelGGL((k_lock_stage<TX, 2>), dim3((unsigned)nt), dim3(TX), lds_stage, st, a, scs, tiles, p, apply_end);
+    // More tiles than CUs: the stage is bound by its FP64 instructions and the
+    // bounded fluxes pay for their spill at 168 registers (96 tubes of 256 to
+    // 4096 cells, 600 tiles: stages 15.8 and 18.9 -> 14.7 and 17.9 us).  Fewer
+    // tiles are bound by latency (a sweep of those took 1.05 times as long).
+    const bool bf = (long long)nt * TX > 256 * kCUs;
+    const auto f = istep == 1 ? (bf ? k_lock_stage<TX, 1, true> : k_lock_stage<TX, 1, false>)
+                              : (bf ? k_lock_stage<TX, 2, true> : k_lock_stage<TX, 2, false>);
+    hipLaunchKernelGGL(f, dim3((unsigned)nt), dim3(TX), lds_stage, st, a, scs, tiles, p, apply_end);
   };
   return PIP_OK;
 }

@@ -11,6 +11,7 @@ from pip_amd import problems
 from pip_amd._lib import check, lib
 from pip_amd.adjoint import TwoFluidRun
 from pip_amd.config import PIPConfig
+from pip_amd.ensemble import Ensemble
 from pip_amd.solver import PIPSolver
 from tests.util import interior
 
@@ -190,3 +191,28 @@ def test_adjoint_gathers(nx, ny, bnd):
     for g, h in ((lam, lam_h), (lam_ac, lam_ac_h)):
         assert np.abs(g.cpu().numpy() - h).max() <= 1e-13 * np.abs(h).max()
     s.close()
+
+
+@pytest.mark.parametrize("extra", [0, 1])
+@pytest.mark.parametrize("tile", [64, 128])
+def test_ensemble_tubes_by_tile_count(tile, extra):
+    """1-D ensembles of 65,536 / tile tiles (general fluxes) and of one more
+    (bounded ones), a member beyond the bounded range among them."""
+    tc, nt = tile - 1, 65536 // tile
+    members = []
+    for nx in ((nt - 12) // 2 * tc, 4 * tc, (nt - 12) // 2 * tc, 7 * tc + 5 + extra * tc):
+        cfg, uh, um, _ = problems.brio_wu(nx)
+        members.append((cfg, uh, um))
+    cfg, uh, um = members[1]
+    big = um * 2.0 ** 104
+    big[5:8] = um[5:8] * 2.0 ** 52
+    members[1] = cfg.replace(col=cfg.col * 2.0 ** -104), uh * 2.0 ** 104, big
+    e = Ensemble(members, tend=1.0e30, max_steps=3, tile=tile)
+    e.set_mode("lockstep")
+    e.run()
+    for m, (cfg, uh, um) in enumerate(members):
+        o = Oracle(cfg, uh, um, None)
+        o.run(nsteps=3)
+        for g, w in zip(e.state(m), o.state()):
+            assert np.array_equal(interior(g, cfg), interior(w, cfg))
+    e.close()
