@@ -114,8 +114,9 @@ int pip_device_state(pip_ctx *ctx, double **U, double **ac);
 int pip_get_stream(pip_ctx *ctx, void **stream);
 /* Stage-kernel tile shape (autotuner): 16x15, 32x7, 32x15, 64x7, 32x8 or
  * 16x7 cells per workgroup.  A context starts with 16x7 on grids of at most
- * 256 such tiles and 16x15 on others; where at most 256 of the set 16x7 or
- * 16x15 tiles cover the grid, each takes eight waves instead of two or four. */
+ * 256 such tiles and on those of more than 8192 tiles of 16x15, and with 16x15
+ * on others; where at most 256 of the set 16x7 or 16x15 tiles cover the grid,
+ * each takes eight waves instead of two or four. */
 int pip_set_tile(pip_ctx *ctx, int tx, int ty);
 /* Bit s-1 of stage_mask set: SSP-RK stage s takes the two fluids one after
  * the other in a tile of nvar_m planes (three workgroups per CU; tiles 16x15,

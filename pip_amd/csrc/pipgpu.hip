@@ -507,6 +507,13 @@ int pip_create(const pip_cfg* cfg, pip_ctx** out) {
   // grids of at most one 16x7 tile per CU take those (launch_stage_tile's split
   // kernel), others 16x15
   if (cfg->ndim == 2 && one_round(c->nx, c->ny, 16, 7)) c->ty = 7;
+  // Grids of at least 16 rounds of two 16x15 workgroups per CU as well: four
+  // workgroups of two waves wait at their barriers for fewer others, and the
+  // halo that they read more of is in L2.  us per step, 16x15 and 16x7:
+  // Orszag-Tang 1024^2 265 / 266, 1500^2 603 / 582, 2048^2 1109 / 1056; KH + IR
+  // 1200^2 475 / 469, 2048^2 1346 / 1303.  Below, the last round decides
+  // (Orszag-Tang 400^2 60 / 69).
+  if (cfg->ndim == 2 && (long long)((c->nx + 15) / 16) * ((c->ny + 14) / 15) > 16 * 2 * kCUs) c->ty = 7;
   // by the 16x7 (127-cell) tiles, whatever tile is set: the set count is fixed
   // for the context
   c->nred = red_sets(cfg->ndim == 2 ? (long long)((c->nx + 15) / 16) * ((c->ny + 6) / 7) : (c->nx + 126) / 127);

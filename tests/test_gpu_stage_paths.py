@@ -216,3 +216,14 @@ def test_ensemble_tubes_by_tile_count(tile, extra):
         for g, w in zip(e.state(m), o.state()):
             assert np.array_equal(interior(g, cfg), interior(w, cfg))
     e.close()
+
+
+@pytest.mark.parametrize("extra", [0, 1])
+@pytest.mark.parametrize("flow", ["orszag_tang", "kelvin_helmholtz"])
+def test_default_tile_of_large_grids(flow, extra):
+    """8192 tiles of 16x15 (those) and more (16x7), the last column partial."""
+    nx, ny = 52, 15 * 2048 + extra
+    cfg, uh, um, _ = cut(flow, nx, 64)
+    rows = np.arange(ny + 4) % 64 + 2
+    cfg = cfg.replace(ny=ny, ymax=cfg.ymin + ny * cfg.dy)
+    same_as_oracle(cfg, uh[:, rows].copy(), um[:, rows].copy(), None, nsteps=2)
