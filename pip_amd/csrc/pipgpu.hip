@@ -706,10 +706,9 @@ static int fused_steps(pip_ctx* c, int n, double* hist, const std::function<void
 
 int pip_run_solver(pip_ctx* c) {
   if (!c) return fail(PIP_ERR_ARG, "null context");
-  TRY(set_loop(c, 1.0e300, (long long)1 << 62, 1, -1));
-  TRY(run_stages(c, 0, c->ion_pot));
-  TRY(set_loop(c, 1.0e300, (long long)1 << 62, -1, 1));  // ion_pot now defined
-  return PIP_OK;
+  // ion_pot is defined from here on: only the cfl calls after the stages ask
+  TRY(set_loop(c, 1.0e300, (long long)1 << 62, 1, 1));
+  return run_stages(c, 0, c->ion_pot);
 }
 
 static int loop_top(pip_ctx* c, double tend, long long nmax) {
