@@ -671,7 +671,7 @@ static int run_stages(pip_ctx* c, int epi_last, double* ion_out) {
 // us): on the split grids and while the 16x15 tiles are one round of two
 // workgroups per CU.  Every workgroup pays for it again: us per step, folded
 // and not, Orszag-Tang 300^2 41.0 / 42.3, 400^2 58.0 / 58.5, 700^2 137.3 / 136.3,
-// KH + IR 2048^2 1455 / 1419.
+// KH + IR 2048^2 1455 / 1419 (1346 now, 1303 on 16x7 tiles).
 static bool fold_steps(const pip_ctx* c) {
   if (split_stages(c)) return true;
   return c->arith == PIP_ARITH_EXACT && !c->two_pass && c->cfg.ndim == 2 &&
