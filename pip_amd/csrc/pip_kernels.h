@@ -110,7 +110,7 @@ struct StageArgs {
   DevScalars* sc;
   RedSlot* red;           // reduction slot sets, nred (a power of two) in use
   int nred;
-  int fold;               // split kernel, stage 1: apply the end of the step before (fin) first
+  int fold;               // k_stage and k_stage_split, stage 1: apply the end of the step before (fin) first
   FinArgs fin;
   int ix, jx, nx, ny;
   long long N;            // plane stride ix*jx
@@ -375,6 +375,8 @@ struct StepLoads {
     st = load_state(a.fold ? a.fin.src : a.sc);
     if (a.fold) slot = load_slot(a.fin.src_red, a.nred, a.fin.flag_ir);
   }
+  // The run is on (before the end of the step before: begin_step asks again).
+  __device__ __forceinline__ bool running() const { return REPLAY || st.active != 0; }
   __device__ __forceinline__ StepNow begin_step(const StageArgs& a) {
     if (REPLAY) return StepNow{a.dtc[0], a.dtc[1], a.epi, true};
     if (a.fold) {
@@ -491,11 +493,12 @@ struct TileGeom {
 // cell's dt terms when epi >= 1.
 // step() is asked for the step's {dt, cmax, epi, active} once the cells' loads
 // have been issued (its own loads then wait beside them); a tile of an inactive
-// run ends there.
+// run ends there.  running false: it is known to be inactive, and nothing is
+// loaded.
 template <int NDIM, int NV, bool IR, bool EXT, int TX, int TY, int NT, int MODE = STAGE_PLAIN, bool BF = NDIM == 2,
           class Step>
 __device__ __forceinline__ bool stage_tile(const StageArgs& a, Step step, int i0, int j0, double* smem, RoundOut& r,
-                                           int& nanflag) {
+                                           int& nanflag, bool running = true) {
   using G = TileGeom<NDIM, NV, TX, TY>;
   constexpr int NVT = G::NVT;
   constexpr int HX = G::HX;
@@ -531,7 +534,7 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, Step step, int i0
   constexpr int NRX = (NDIM == 2) ? 4 * TX : 0;  // ring cells above and below
   constexpr int NR = NRX + 4 * TY;               // ... and at the sides
   // past the grid's edge a tile still needs the ghost cells there
-  const bool inside = (tid < TX * TY) && ci < a.ix && cj < a.jx;
+  const bool inside = running && (tid < TX * TY) && ci < a.ix && cj < a.jx;
   // (in 2-D; 1-D tiles read it again, as the 26 registers across the solvers
   // would cost the third workgroup of a CU)
   constexpr bool KEEP = NDIM == 2;
@@ -545,7 +548,7 @@ __device__ __forceinline__ bool stage_tile(const StageArgs& a, Step step, int i0
   const int rx = (tid < NRX) ? 2 + tid % TX : (rk < 2 ? rk : TX + rk);
   const int ry = (tid < NRX) ? (rk < 2 ? rk : TY + rk) : OY + (tid - NRX) / 4;
   const int gi = i0 + rx, gj = (NDIM == 2) ? j0 + ry : 0;
-  const bool on_ring = tid < NR && gi < a.ix && gj < a.jx;
+  const bool on_ring = running && tid < NR && gi < a.ix && gj < a.jx;
   double ring[NVT];
   if (on_ring) {
 #pragma unroll
@@ -719,6 +722,18 @@ __global__ void __launch_bounds__(NT, NDIM == 1 ? 3 : 2) k_stage(StageArgs a) {
   extern __shared__ double smem[];
   constexpr bool REPLAY = (MODE == STAGE_REPLAY);
   StepLoads<REPLAY> loads(a);
+  // A run that has stopped leaves the chunk's other launches here.  The
+  // arguments that the tile's loads need are asked for first, so that they
+  // arrive with the flag: a return ahead of them cost a running step of 600^2
+  // 1.5 % (a third wait in a row), this one 0.4 %.  us per step of a stopped
+  // run, without and with it: Orszag-Tang 1024^2 52 / 9, KH + IR 2048^2 315 / 25
+  // (their running steps 259 and 1293).  With fold the step's end is still to
+  // be passed on; those tiles only skip their loads (300^2: 7.9 / 4.7).
+  if (!REPLAY) {
+    asm volatile("" ::"s"(a.Uin), "s"(a.N), "s"(a.ix), "s"(a.jx), "s"(a.nx), "s"(a.ny), "s"(a.xcd_remap),
+                 "s"(gridDim.x));
+    if (!a.fold && !loads.running()) return;
+  }
   const int ntx = (a.nx + TX - 1) / TX;
   int bid = blockIdx.x;
   if (a.xcd_remap) bid = xcd_tile(bid, gridDim.x);
@@ -734,7 +749,7 @@ __global__ void __launch_bounds__(NT, NDIM == 1 ? 3 : 2) k_stage(StageArgs a) {
         active = now.active;
         return now;
       },
-      i0, j0, smem, r, nanflag);
+      i0, j0, smem, r, nanflag, loads.running());
   if (!REPLAY && a.epi >= 1 && active) {
     __syncthreads();
     block_reduce_store<NT, IR>(r, nanflag, valid, a.red[blockIdx.x & (a.nred - 1)].v, smem);
@@ -802,8 +817,9 @@ __global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageA
   const int ti = t % TX, tj = t / TX;
   const int ci = i0 + ti + 2, cj = (NDIM == 2) ? j0 + tj + 2 : 0;
   const long long oc = (long long)cj * ix + ci;
-  const bool inside = cells && t < NC && ci < a.ix && cj < a.jx;
-  const bool valid = cells && t < NC && i0 + ti < a.nx && j0 + tj < a.ny;
+  const bool running = loads.running();
+  const bool inside = running && cells && t < NC && ci < a.ix && cj < a.jx;
+  const bool valid = running && cells && t < NC && i0 + ti < a.nx && j0 + tj < a.ny;
 
   // ---- load
   double own[NV], base[NV], other[NV];  // this fluid's cell, its stage base; for the neutrals the plasma's cell
@@ -814,7 +830,7 @@ __global__ void __launch_bounds__(NDIM == 2 ? 512 : 256, 2) k_stage_split(StageA
   const int rx = (t < NRX) ? 2 + t % TX : (rk < 2 ? rk : TX + rk);
   const int ry = (t < NRX) ? (rk < 2 ? rk : TY + rk) : OY + (t - NRX) / 4;
   const int gi = i0 + rx, gj = (NDIM == 2) ? j0 + ry : 0;
-  const bool on_ring = rest && t < NR && gi < a.ix && gj < a.jx;
+  const bool on_ring = running && rest && t < NR && gi < a.ix && gj < a.jx;
   auto load = [&](auto fl) {
     constexpr int FL = decltype(fl)::value, NFL = FL ? 5 : NV, OFF = FL ? NV : 0;
     if (inside) {
@@ -1305,6 +1321,10 @@ __global__ void __launch_bounds__(64) k_finalize(FinArgs f) {
   DevScalars* sc = f.sc;
   if (f.mode == 1) {
     StepState s = load_state(f.src);
+    if (!s.active && f.src == sc) {  // stopped before: nothing to end or to pass on, the slots are as reset
+      if (f.hist && threadIdx.x == 0) record_dt(s, f.hist, f.hist_k);
+      return;
+    }
     if (s.active) s = step_end(s, combine_slots(load_slot(f.src_red, f.nred, f.flag_ir), f.nred, f.flag_ir), f);
     if ((int)threadIdx.x < f.nred) {
       f.red[threadIdx.x] = red_slot_init();
