@@ -116,10 +116,11 @@ PIP_HD bool hllc_flux_b(const double* v_l, const double* v_r, double gm, double 
   const double den = v_r[0] * ar - v_l[0] * al;
   const double sm = quob(mr * ar - ml * al + v_l[4] - v_r[4], den, qrcp(den));
   const double dl = sl - sm, dr = sr - sm;
-  // thl, thm, thr exactly 0 or 1, and neither star state divides by zero
-  const double hb = 0.5 * kEpsi;
-  const bool ok = (sm <= 0.0 || sm >= hb) && (sl <= 0.0 || sl >= hb) && (sr <= 0.0 || sr >= hb) && dl != 0.0 &&
-                  dr != 0.0;
+  // thl, thm, thr exactly 0 or 1, and neither star state divides by zero or
+  // infinity (den passes through zero in supersonic flow)
+  const double hb = 0.5 * kEpsi, dd = fabs(dl * dr);
+  const bool ok = (sm <= 0.0 || sm >= hb) && (sl <= 0.0 || sl >= hb) && (sr <= 0.0 || sr >= hb) && dd > 0.0 &&
+                  dd < HUGE_VAL;
   if (!ok) return false;
   const double pr_m = sm * v_l[0] * al - ml * al + v_l[4];
   // the side whose states the flux is made of: left of the contact or, in a
