@@ -7,9 +7,9 @@
 // Face states lie between cell values, so no intermediate of these functions
 // overflows, no divisor is subnormal, and a value differs from that of the
 // general function in the sign of a zero at most.  Where a function cannot
-// vouch for that (a divisor that came out zero, a state inside one of HLLC's
-// switch bands) it says so and the caller takes the general function for that
-// face.  The stage kernels are bound by FP64 VALU issue (4 cycles a wave
+// vouch for that (a divisor that came out zero or infinite, an outer wave of
+// HLLC's inside its switch band) it says so and the caller takes the general
+// function for that face.  The stage kernels are bound by FP64 VALU issue (4 cycles a wave
 // instruction, 16 for v_rcp_f64 and v_rsq_f64), so every identity below is
 // one that removes instructions without changing a bit:
 //   - a product with a power of two is exact, so k x + y is one fma;
@@ -18,7 +18,7 @@
 //     no zero / infinity test in the square root;
 //   - min(max(X, Y), 0) and min(X, Y) give minmod(X, Y) as a median;
 //   - HLLC's switches |S| + S over max(2 S, eps) are exactly 0 or 1 outside
-//     (0, eps / 2), so one side's flux and star state are enough;
+//     (0, eps / 2), so one side's flux and star state are enough there;
 //   - 1 / sqrt(x) comes from the square root's own iteration.
 #pragma once
 
@@ -101,7 +101,14 @@ PIP_HD bool bounded_cell(const double* v, int nv) {
 }
 
 // hllc_flux for bounded states, handed out as put(n, flux); false: not
-// covered (take hllc_flux).  rg1 = 1 / (gm - 1).
+// covered (take hllc_flux).  rg1 = 1 / (gm - 1).  Near rest, half of the
+// contact speeds lie in (0, eps / 2), where the switch is a fraction and both
+// star states count: such a wave forms its fluxes once for either side and
+// blends them.  us per step with those faces left to the general function,
+// which solves them again, with the blend, and with the general function
+// alone, velocities up to 1e-13: 96 tubes 38.9 / 35.3 / 35.4, 300^2 47.4 / 43.2 /
+// 56.0, 1024^2 326 / 290 / 355.  One loop for both kinds of wave cost moving
+// flows 1.4 %.
 template <class Put>
 PIP_HD bool hllc_flux_b(const double* v_l, const double* v_r, double gm, double rg1, Put put) {
   const double ml = v_l[0] * v_l[1], mr = v_r[0] * v_r[1];
@@ -116,36 +123,54 @@ PIP_HD bool hllc_flux_b(const double* v_l, const double* v_r, double gm, double 
   const double den = v_r[0] * ar - v_l[0] * al;
   const double sm = quob(mr * ar - ml * al + v_l[4] - v_r[4], den, qrcp(den));
   const double dl = sl - sm, dr = sr - sm;
-  // thl, thm, thr exactly 0 or 1, and neither star state divides by zero or
+  // thl, thr exactly 0 or 1, and neither star state divides by zero or
   // infinity (den passes through zero in supersonic flow)
   const double hb = 0.5 * kEpsi, dd = fabs(dl * dr);
-  const bool ok = (sm <= 0.0 || sm >= hb) && (sl <= 0.0 || sl >= hb) && (sr <= 0.0 || sr >= hb) && dd > 0.0 &&
-                  dd < HUGE_VAL;
+  const bool ok = (sl <= 0.0 || sl >= hb) && (sr <= 0.0 || sr >= hb) && dd > 0.0 && dd < HUGE_VAL;
   if (!ok) return false;
   const double pr_m = sm * v_l[0] * al - ml * al + v_l[4];
   // the side whose states the flux is made of: left of the contact or, in a
   // supersonic flow (thl = 1, or thr = 1: that side's own flux), upstream
   const bool upl = sl > 0.0, upr = sr <= 0.0;
-  const bool left = upl || (sm > 0.0 && !upr);
-  const double r0 = left ? v_l[0] : v_r[0], r1 = left ? v_l[1] : v_r[1];
-  const double r2 = left ? v_l[2] : v_r[2], r3 = left ? v_l[3] : v_r[3];
-  const double pr = left ? v_l[4] : v_r[4], ri = left ? ra : rb;
-  const double vn = left ? vn_l : vn_r, d = left ? dl : dr, as = left ? al : ar;
-  double s = left ? sl : sr;
-  const double m1 = r0 * r1, m2 = r0 * r2, m3 = r0 * r3;
-  const double en = fma2(0.5, r0 * ((r1 * r1 + r2 * r2) + r3 * r3), quob(pr, gm - 1.0, rg1));
-  const double rd = qrcp(d);
-  const double st0 = quob(r0 * as, d, rd);
-  const double st1 = st0 * sm;
-  const double st2 = quob(st0 * m2, r0, ri);
-  const double st3 = quob(st0 * m3, r0, ri);
-  const double st4 = quob(as * en - pr * vn + pr_m * sm, d, rd);
-  if (upl || upr) s = 0.0;
-  put(0, m1 + s * (st0 - r0));
-  put(1, (pr + quob(m1 * m1, r0, ri)) + s * (st1 - m1));
-  put(2, quob(m1 * m2, r0, ri) + s * (st2 - m2));
-  put(3, quob(m1 * m3, r0, ri) + s * (st3 - m3));
-  put(4, quob(m1 * (en + pr), r0, ri) + s * (st4 - en));
+  auto side = [&](bool left, auto out) {
+    const double r0 = left ? v_l[0] : v_r[0], r1 = left ? v_l[1] : v_r[1];
+    const double r2 = left ? v_l[2] : v_r[2], r3 = left ? v_l[3] : v_r[3];
+    const double pr = left ? v_l[4] : v_r[4], ri = left ? ra : rb;
+    const double vn = left ? vn_l : vn_r, d = left ? dl : dr, as = left ? al : ar;
+    double s = left ? sl : sr;
+    const double m1 = r0 * r1, m2 = r0 * r2, m3 = r0 * r3;
+    const double en = fma2(0.5, r0 * ((r1 * r1 + r2 * r2) + r3 * r3), quob(pr, gm - 1.0, rg1));
+    const double rd = qrcp(d);
+    const double st0 = quob(r0 * as, d, rd);
+    const double st1 = st0 * sm;
+    const double st2 = quob(st0 * m2, r0, ri);
+    const double st3 = quob(st0 * m3, r0, ri);
+    const double st4 = quob(as * en - pr * vn + pr_m * sm, d, rd);
+    if (upl || upr) s = 0.0;
+    out(0, m1 + s * (st0 - r0));
+    out(1, (pr + quob(m1 * m1, r0, ri)) + s * (st1 - m1));
+    out(2, quob(m1 * m2, r0, ri) + s * (st2 - m2));
+    out(3, quob(m1 * m3, r0, ri) + s * (st3 - m3));
+    out(4, quob(m1 * (en + pr), r0, ri) + s * (st4 - en));
+  };
+  const bool one = upl || (sm > 0.0 && !upr);
+  const bool both = sm > 0.0 && sm < hb && !upl && !upr;  // thm is a fraction
+  if (!wave_any(both)) {
+    side(one, put);
+    return true;
+  }
+  // the right side's flux first, then the left one's
+  const double thm = both ? qdiv(sm + sm, kEpsi) : 1.0;
+  double f_r[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+  for (int pass = 0; pass < 2; pass++) {
+    double f[5];
+    side(both ? pass == 1 : one, [&](int n, double x) { f[n] = x; });
+    for (int n = 0; n < 5; n++) {
+      if (pass == 0) f_r[n] = f[n];
+      else put(n, thm * f[n] + (1.0 - thm) * f_r[n]);
+    }
+  }
   return true;
 }
 
