@@ -441,7 +441,8 @@ __device__ __forceinline__ void face_flux(const double* v, double* f, const Phys
 #pragma unroll
     for (int n = 0; n < NFL; n++) {
       const double* c = v + perm(n) * PV;
-      face_states(c[0], c[ST], c[2 * ST], c[3 * ST], vl[n], vr[n]);
+      if (n == 0 || n == 4) face_states<true>(c[0], c[ST], c[2 * ST], c[3 * ST], vl[n], vr[n]);
+      else face_states(c[0], c[ST], c[2 * ST], c[3 * ST], vl[n], vr[n]);
     }
     vl[0] = dmax(vl[0], ph.ro_lim);
     vr[0] = dmax(vr[0], ph.ro_lim);

@@ -5,14 +5,19 @@
 // (2^-100, 2^100) and the other variables below 2^100 in magnitude (no NaN,
 // no infinity): stage_tile checks it once per cell while it loads the tile.
 // Face states lie between cell values, so no intermediate of these functions
-// overflows, no divisor is subnormal, and a value differs from that of the
-// general function in the sign of a zero at most.  Where a function cannot
+// overflows, no divisor is subnormal, and values equal those of the general
+// function; the sign of a zero may differ (the median of slopes, and the normal
+// field and the blends without the general form's terms in +0).  No later
+// operation tells such zeros apart: none is divided by, and the one copysign,
+// of the normal field, is reached only where that is not zero.  Where a function cannot
 // vouch for that (a divisor that came out zero or infinite, an outer wave of
 // HLLC's inside its switch band) it says so and the caller takes the general
 // function for that face.  The stage kernels are bound by FP64 VALU issue (4 cycles a wave
 // instruction, 16 for v_rcp_f64 and v_rsq_f64), so every identity below is
-// one that removes instructions without changing a bit:
-//   - a product with a power of two is exact, so k x + y is one fma;
+// one that removes instructions without changing a value:
+//   - a product with a power of two is exact above the subnormal numbers, so
+//     k x + y is one fma where the product is not subnormal or is added to a
+//     pressure or energy (at least 2^-100, which no subnormal changes);
 //   - max and the rounded square root commute (both are monotonic);
 //   - finite non-zero divisors need no v_div_fixup_f64, positive arguments
 //     no zero / infinity test in the square root;
@@ -75,10 +80,16 @@ PIP_HD double qdivb(double n, double d) { return quob(n, d, qrcp(d)); }
 PIP_HD double minmod_med(double X, double Y) { return dmax(dmin(X, Y), dmin(dmax(X, Y), 0.0)); }
 
 // The face states of get_Side (HLL_rot.f90:33-51) from the stencil a0..a3.
+// POS: of a bounded tile's density or pressure, where half a slope is exact.
+// Velocities and fields may be subnormal (ahead of a front), and half a
+// subnormal slope rounds: one fma there put 1-D states 1e-323 off what the
+// general face states give (its products cost a step 0.2 to 1 %).
+template <bool POS = false>
 PIP_HD void face_states(double a0, double a1, double a2, double a3, double& vl, double& vr) {
   const double d0 = a1 - a0, d1 = a2 - a1, d2 = a3 - a2;
-  vl = fma2(0.5, minmod_med(d1, d0), a1);
-  vr = fma2(-0.5, minmod_med(d2, d1), a2);
+  const double ml = minmod_med(d1, d0), mr = minmod_med(d2, d1);
+  vl = POS ? fma2(0.5, ml, a1) : a1 + 0.5 * ml;
+  vr = POS ? fma2(-0.5, mr, a2) : a2 - 0.5 * mr;
 }
 
 // Any active lane of the wave (host: this call).
