@@ -146,8 +146,10 @@ int pip_set_arith(pip_ctx *ctx, int mode);
  * range of tiles (neighbouring halos in one L2; a 2-D context starts with
  * it); 0: row-major (autotuner). */
 int pip_set_xcd_remap(pip_ctx *ctx, int on);
-/* Average device time (ms) of the last timed enqueue of the dominant kernel;
- * measured with hipEvents on the context's stream. */
+/* Device time (ms) of nsteps steps as pip_advance queues them, measured with
+ * hipEvents on the context's stream.  With ms_stage1 or ms_stage2, also that
+ * of their first and second stages; the events between the launches then add
+ * about 3.5 us each (three a step) to the total.  t_order = 2. */
 int pip_time_steps(pip_ctx *ctx, int nsteps, double *ms_total, double *ms_stage1, double *ms_stage2);
 
 /* ---- discrete adjoint (no counterpart in the reference: PIP has no

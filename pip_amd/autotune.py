@@ -69,7 +69,7 @@ def tune_stage(make_solver, cfg, steps: int = 20, use_cache: bool = True, arith:
         s = make_solver(cand)
         s.enqueue(3)
         s.sync()
-        ev = s.time_steps(steps)
+        ev = s.time_steps(steps, stages=False)
         timings["x".join(str(v) for v in cand)] = ev["total_ms"] / steps
         s.close()
     best = min(timings, key=timings.get)

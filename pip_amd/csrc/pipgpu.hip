@@ -680,8 +680,10 @@ static bool fold_steps(const pip_ctx* c) {
 
 // n steps of the loop; stage(k, s, a) may redirect stage s of step k.  hist:
 // record {dt, cmax} of steps 1..n-1 (step 0's is there).  A chunk ends on
-// k_finalize whether or not its steps are folded.
-static int fused_steps(pip_ctx* c, int n, double* hist, const std::function<void(int, int, StageArgs&)>& stage) {
+// k_finalize whether or not its steps are folded.  marks: events to record
+// before each stage of a step and after its last, t_order + 1 a step.
+static int fused_steps(pip_ctx* c, int n, double* hist, const std::function<void(int, int, StageArgs&)>& stage,
+                       hipEvent_t* marks = nullptr) {
   const bool fold = fold_steps(c);
   const int T = c->cfg.t_order;
   for (int k = 0; k < n; k++) {
@@ -697,8 +699,10 @@ static int fused_steps(pip_ctx* c, int n, double* hist, const std::function<void
         a.fin = fin_args(c, 1, 0, hist, k, p ^ 1);
       }
       if (stage) stage(k, s, a);
+      if (marks) HIPCHK(hipEventRecord(*marks++, c->stream));
       TRY(launch_stage(c, a));
     }
+    if (marks) HIPCHK(hipEventRecord(*marks++, c->stream));
     if (!fold || k + 1 == n) TRY(launch_finalize(c, 1, 0, (k + 1 < n) ? hist : nullptr, k + 1, p));
   }
   return PIP_OK;
@@ -939,44 +943,39 @@ int pip_set_xcd_remap(pip_ctx* c, int on) {
 
 int pip_time_steps(pip_ctx* c, int nsteps, double* ms_total, double* ms_stage1, double* ms_stage2) {
   if (!c) return fail(PIP_ERR_ARG, "null context");
+  if (nsteps < 0) return fail(PIP_ERR_ARG, "nsteps < 0");
   if (c->cfg.t_order != 2) return fail(PIP_ERR_UNSUPPORTED, "timing helper covers t_order = 2");
   if (c->top_pending) TRY(loop_top(c, 1.0e300, (long long)1 << 62));
-  const int NE = 3 * nsteps + 1;
-  hipEvent_t* ev = new hipEvent_t[NE];
-  for (int k = 0; k < NE; k++) HIPCHK(hipEventCreate(&ev[k]));
-  HIPCHK(hipEventRecord(ev[0], c->stream));
-  int rc = PIP_OK;
-  for (int k = 0; k < nsteps && rc == PIP_OK; k++) {
-    StageArgs a1 = stage_args(c, 1, c->U, c->U, c->U1, 0, nullptr);
-    rc = launch_stage(c, a1);
-    if (rc != PIP_OK) break;
-    HIPCHK(hipEventRecord(ev[3 * k + 1], c->stream));
-    StageArgs a2 = stage_args(c, 2, c->U1, c->U, c->U, 2, nullptr);
-    rc = launch_stage(c, a2);
-    if (rc != PIP_OK) break;
-    HIPCHK(hipEventRecord(ev[3 * k + 2], c->stream));
-    rc = launch_finalize(c, 1, 0);
-    if (rc != PIP_OK) break;
-    HIPCHK(hipEventRecord(ev[3 * k + 3], c->stream));
-  }
+  struct Events {  // [0], [1]: start and end; then the marks
+    std::vector<hipEvent_t> e;
+    ~Events() {
+      for (hipEvent_t x : e)
+        if (x) (void)hipEventDestroy(x);
+    }
+  } ev;
+  const bool stages = ms_stage1 || ms_stage2;
+  ev.e.assign(2 + (stages ? 3 * (size_t)nsteps : 0), nullptr);
+  for (auto& x : ev.e) HIPCHK(hipEventCreate(&x));
+  hipEvent_t* marks = ev.e.data() + 2;
+  HIPCHK(hipEventRecord(ev.e[0], c->stream));
+  const int rc = fused_steps(c, nsteps, nullptr, nullptr, stages ? marks : nullptr);
+  HIPCHK(hipEventRecord(ev.e[1], c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
-  double t1 = 0, t2 = 0, tt = 0;
+  c->top_pending = true;
+  if (rc != PIP_OK) return rc;
+  double t1 = 0, t2 = 0;
   float ms;
-  for (int k = 0; k < nsteps && rc == PIP_OK; k++) {
-    HIPCHK(hipEventElapsedTime(&ms, ev[3 * k], ev[3 * k + 1]));
+  for (int k = 0; stages && k < nsteps; k++) {
+    HIPCHK(hipEventElapsedTime(&ms, marks[3 * k], marks[3 * k + 1]));
     t1 += ms;
-    HIPCHK(hipEventElapsedTime(&ms, ev[3 * k + 1], ev[3 * k + 2]));
+    HIPCHK(hipEventElapsedTime(&ms, marks[3 * k + 1], marks[3 * k + 2]));
     t2 += ms;
   }
-  HIPCHK(hipEventElapsedTime(&ms, ev[0], ev[NE - 1]));
-  tt = ms;
-  for (int k = 0; k < NE; k++) (void)hipEventDestroy(ev[k]);
-  delete[] ev;
-  if (ms_total) *ms_total = tt;
+  HIPCHK(hipEventElapsedTime(&ms, ev.e[0], ev.e[1]));
+  if (ms_total) *ms_total = ms;
   if (ms_stage1) *ms_stage1 = t1;
   if (ms_stage2) *ms_stage2 = t2;
-  c->top_pending = true;
-  return rc;
+  return PIP_OK;
 }
 
 }  // extern "C"

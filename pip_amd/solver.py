@@ -179,11 +179,16 @@ class PIPSolver:
         check(lib().pip_set_arith(self.h, ARITH[arith]))
         self.arith = arith
 
-    def time_steps(self, nsteps: int):
+    def time_steps(self, nsteps: int, stages: bool = True):
+        """Device time of nsteps steps; stages: of their two stages as well
+        (whose events lengthen the total)."""
         tt, t1, t2 = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()
-        check(lib().pip_time_steps(self.h, int(nsteps), ctypes.byref(tt), ctypes.byref(t1),
-                                   ctypes.byref(t2)))
-        return dict(total_ms=tt.value, stage1_ms=t1.value, stage2_ms=t2.value)
+        check(lib().pip_time_steps(self.h, int(nsteps), ctypes.byref(tt), ctypes.byref(t1) if stages else None,
+                                   ctypes.byref(t2) if stages else None))
+        out = dict(total_ms=tt.value)
+        if stages:
+            out.update(stage1_ms=t1.value, stage2_ms=t2.value)
+        return out
 
     def device_state(self):
         U = ctypes.c_void_p()
