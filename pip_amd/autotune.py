@@ -35,9 +35,14 @@ def _save(d):
     json.dump(d, open(CACHE, "w"), indent=1)
 
 
+# Changes with the kernels and with what is timed: a choice cached for others is
+# not taken.
+VERSION = 3
+
+
 def stage_key(cfg, arith: str = "exact") -> str:
-    key = (f"stage2:{cfg.ndim}:{cfg.nx}x{cfg.ny}:nv{cfg.nvar_m}:ir{cfg.flag_ir}:ac{int(cfg.ac_field)}"
-           f":col{cfg.flag_col}:imp{cfg.flag_pip_imp}:twopass")
+    key = (f"stage{VERSION}:rk{cfg.t_order}:{cfg.ndim}:{cfg.nx}x{cfg.ny}:nv{cfg.nvar_m}:ir{cfg.flag_ir}"
+           f":ac{int(cfg.ac_field)}:col{cfg.flag_col}:imp{cfg.flag_pip_imp}:twopass")
     return key if arith == "exact" else key + ":" + arith
 
 
@@ -83,7 +88,7 @@ def tune_ensemble(ens, key: str, use_cache: bool = True):
     """Time the whole ensemble for each launch mode and workgroup width;
     sets the fastest and returns ((mode, width), timings)."""
     cache = _load()
-    key = key + ":modes"
+    key = f"{key}:modes{VERSION}"
     if use_cache and key in cache:
         mode, tx = cache[key]["best"]
         ens.set_mode(mode)
