@@ -259,6 +259,10 @@ int pip_ens_destroy(pip_ens *e);
  * conversions and cfl terms use (host arrays of count doubles; synchronous;
  * allocates). */
 int pip_check_arith(const double *n, const double *d, double *q, double *r, long long count);
+/* The same for the sequences of the bounded-state fluxes (finite n, positive
+ * finite d): q[k] = n[k] / d[k], r[k] = sqrt(d[k]), s[k] = n[k] / sqrt(d[k]). */
+int pip_check_arith_bounded(const double *n, const double *d, double *q, double *r, double *s,
+                            long long count);
 
 const char *pip_last_error(void);
 const char *pip_version(void);

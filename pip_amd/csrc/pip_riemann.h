@@ -43,8 +43,10 @@ __device__ __forceinline__ double quob(double n, double d, double r) {
 }
 #endif
 // sqrt(x) for positive finite x: qsqrt without its zero / infinity test;
-// sqrt_rcp also gives qrcp of the root: h = 1 / (2 sqrt x) of the iteration is
-// within a few ulp, so one Newton step replaces v_rcp_f64 and the first step.
+// sqrt_rcp also gives a reciprocal of the root: h = 1 / (2 sqrt x) of the
+// iteration is good to about 2^-47 (v_rsq_f64's 2^-24, squared by the step), so
+// one Newton step replaces v_rcp_f64 and its two.  pip_check_arith_bounded runs
+// these sequences beside the IEEE quotient and root.
 __device__ __forceinline__ double sqrtb_h(double x, double& h) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y;

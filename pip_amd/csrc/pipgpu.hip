@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <functional>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -42,6 +43,18 @@ __global__ void k_check_arith(const double* n, const double* d, double* q, doubl
   if (k >= count) return;
   q[k] = qdiv(n[k], d[k]);
   r[k] = qsqrt(n[k]);
+}
+// Those of the bounded fluxes: n / d, sqrt(d) and n / sqrt(d), the last with
+// the reciprocal of the root's own iteration.
+__global__ void k_check_arith_bounded(const double* n, const double* d, double* q, double* r, double* s,
+                                      long long count) {
+  const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= count) return;
+  q[k] = qdivb(n[k], d[k]);
+  r[k] = sqrtb(d[k]);
+  double h;
+  const double g = sqrt_rcp(d[k], h);
+  s[k] = quob(n[k], g, h);
 }
 
 // Work memory of pip_adj_step_noalloc: the face-state adjoint pairs and
@@ -422,31 +435,52 @@ static int set_loop(pip_ctx* c, double tend, long long nmax, int active, int ion
   } while (0)
 
 // ------------------------------------------------------------------ C-ABI
+// Host arrays n and d through launch(grid, n, d, out) to the arrays `outs`,
+// which lie count apart in its out.
+static int check_arith(const char* who, const double* n, const double* d, std::initializer_list<double*> outs,
+                       long long count, const std::function<void(dim3, const double*, const double*, double*)>& launch) {
+  bool arrays = n && d;
+  for (const double* o : outs) arrays = arrays && o;
+  if (count < 0 || count > (1LL << 31) || (count > 0 && !arrays))
+    return fail(PIP_ERR_ARG, std::string(who) + ": bad arguments (0 <= count <= 2^31, non-null arrays)");
+  if (count == 0) return PIP_OK;
+  const size_t b = (size_t)count * sizeof(double);
+  double* buf = nullptr;
+  HIPCHK(hipMalloc(&buf, (2 + outs.size()) * b));
+  hipError_t e = hipMemcpy(buf, n, b, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(buf + count, d, b, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    launch(dim3((unsigned)((count + 255) / 256)), buf, buf + count, buf + 2 * count);
+    e = hipGetLastError();
+  }
+  double* from = buf + 2 * count;
+  for (double* o : outs) {
+    if (e == hipSuccess) e = hipMemcpy(o, from, b, hipMemcpyDeviceToHost);
+    from += count;
+  }
+  const hipError_t ef = hipFree(buf);
+  if (e != hipSuccess) return fail(PIP_ERR_HIP, std::string(who) + ": " + hipGetErrorString(e));
+  if (ef != hipSuccess) return fail(PIP_ERR_HIP, std::string(who) + ": " + hipGetErrorString(ef));
+  return PIP_OK;
+}
+
 extern "C" {
 
 const char* pip_last_error(void) { return g_err.c_str(); }
 
 int pip_check_arith(const double* n, const double* d, double* q, double* r, long long count) {
-  if (count < 0 || count > (1LL << 31) || (count > 0 && !(n && d && q && r)))
-    return fail(PIP_ERR_ARG, "pip_check_arith: bad arguments (0 <= count <= 2^31, non-null arrays)");
-  if (count == 0) return PIP_OK;
-  const size_t b = (size_t)count * sizeof(double);
-  double* buf = nullptr;
-  HIPCHK(hipMalloc(&buf, 4 * b));
-  double *dn = buf, *dd = buf + count, *dq = buf + 2 * count, *dr = buf + 3 * count;
-  hipError_t e = hipMemcpy(dn, n, b, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(dd, d, b, hipMemcpyHostToDevice);
-  if (e == hipSuccess) {
-    const unsigned nb = (unsigned)((count + 255) / 256);
-    hipLaunchKernelGGL(k_check_arith, dim3(nb), dim3(256), 0, 0, dn, dd, dq, dr, count);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipMemcpy(q, dq, b, hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(r, dr, b, hipMemcpyDeviceToHost);
-  const hipError_t ef = hipFree(buf);
-  if (e != hipSuccess) return fail(PIP_ERR_HIP, std::string("pip_check_arith: ") + hipGetErrorString(e));
-  if (ef != hipSuccess) return fail(PIP_ERR_HIP, std::string("pip_check_arith: ") + hipGetErrorString(ef));
-  return PIP_OK;
+  return check_arith("pip_check_arith", n, d, {q, r}, count,
+                     [count](dim3 grid, const double* dn, const double* dd, double* out) {
+                       hipLaunchKernelGGL(k_check_arith, grid, dim3(256), 0, 0, dn, dd, out, out + count, count);
+                     });
+}
+
+int pip_check_arith_bounded(const double* n, const double* d, double* q, double* r, double* s, long long count) {
+  return check_arith("pip_check_arith_bounded", n, d, {q, r, s}, count,
+                     [count](dim3 grid, const double* dn, const double* dd, double* out) {
+                       hipLaunchKernelGGL(k_check_arith_bounded, grid, dim3(256), 0, 0, dn, dd, out, out + count,
+                                          out + 2 * count, count);
+                     });
 }
 const char* pip_version(void) { return "pipgpu 0.1 (gfx950, fp64)"; }
 
