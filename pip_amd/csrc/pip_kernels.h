@@ -1793,30 +1793,32 @@ __device__ __forceinline__ StageArgs ens_stage_args2(const EnsArgs& e, const Ens
 // every cell (ghosts included, as k_round does; pointwise, so one pass makes
 // both rewrites) reduced into the member's slots; the members' scalars.  One
 // workgroup a member took 1.0 ms for the 68,000 cells of a 256^2 member, these
-// take 0.03.
+// take 0.03.  A member's workgroups go over its cells in strides, as the host
+// limits their number (kStartGroups).
 __global__ void __launch_bounds__(256) k_lock_bnd2(EnsArgs e, DevScalars* scs) {
   const int m = blockIdx.y;
   const EnsMember M = e.mem[m];
-  const long long k = (long long)blockIdx.x * 256 + threadIdx.x, N = (long long)M.ix * M.jx;
-  if (k == 0) {
+  const long long N = (long long)M.ix * M.jx;
+  double* U = e.U + M.off;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     const RedSlot r = red_slot_init();
     for (int n = 0; n < RED_N; n++) scs[m].red[n] = r.v[n];
   }
-  if (k >= N) return;
-  const int i = (int)(k % M.ix), j = (int)(k / M.ix);
-  const bool gx = (i < 2 || i >= M.ix - 2), gy = (j < 2 || j >= M.jx - 2);
-  if (!gx && !gy) return;
-  bool fx = false, fy = false;
-  const int si = gx ? src_index(i, M.ix, e.bnd.type[0], e.bnd.type[1], fx) : i;
-  const int sj = gy ? src_index(j, M.jx, e.bnd.type[2], e.bnd.type[3], fy) : j;
-  unsigned msk = 0u;
-  if (fx) msk ^= e.bnd.sym[(i < 2) ? 0 : 1];
-  if (fy) msk ^= e.bnd.sym[(j < 2) ? 2 : 3];
-  double* U = e.U + M.off;
-  const long long src = (long long)sj * M.ix + si;
-  for (int n = 0; n < 14; n++) {
-    const double v = U[n * N + src];
-    U[n * N + k] = ((msk >> n) & 1u) ? -v : v;
+  for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < N; k += (long long)gridDim.x * 256) {
+    const int i = (int)(k % M.ix), j = (int)(k / M.ix);
+    const bool gx = (i < 2 || i >= M.ix - 2), gy = (j < 2 || j >= M.jx - 2);
+    if (!gx && !gy) continue;
+    bool fx = false, fy = false;
+    const int si = gx ? src_index(i, M.ix, e.bnd.type[0], e.bnd.type[1], fx) : i;
+    const int sj = gy ? src_index(j, M.jx, e.bnd.type[2], e.bnd.type[3], fy) : j;
+    unsigned msk = 0u;
+    if (fx) msk ^= e.bnd.sym[(i < 2) ? 0 : 1];
+    if (fy) msk ^= e.bnd.sym[(j < 2) ? 2 : 3];
+    const long long src = (long long)sj * M.ix + si;
+    for (int n = 0; n < 14; n++) {
+      const double v = U[n * N + src];
+      U[n * N + k] = ((msk >> n) & 1u) ? -v : v;
+    }
   }
 }
 
@@ -1824,23 +1826,23 @@ __global__ void __launch_bounds__(256) k_lock_cfl2(EnsArgs e, DevScalars* scs) {
   __shared__ double red_lds[4 * 5];
   const int m = blockIdx.y;
   const EnsMember M = e.mem[m];
-  const long long k = (long long)blockIdx.x * 256 + threadIdx.x, N = (long long)M.ix * M.jx;
+  const long long N = (long long)M.ix * M.jx;
   if ((long long)blockIdx.x * 256 >= N) return;
+  double* U = e.U + M.off;
   RoundOut r = {1.0e300, 0.0, 0.0, 0.0};
-  if (k < N) {
-    double* U = e.U + M.off;
+  for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < N; k += (long long)gridDim.x * 256) {
     double u[14];
 #pragma unroll
     for (int n = 0; n < 14; n++) u[n] = U[n * N + k];
     cfl_cell<9>(u, u + 9, M.gmin_safety, e.ph);
     const double dtc = cfl_cell<9>(u, u + 9, M.gmin_safety, e.ph);
     const int i = (int)(k % M.ix), j = (int)(k / M.ix);
-    if (i >= 2 && i < M.ix - 2 && j >= 2 && j < M.jx - 2) r.dtc = dtc;
-    r.rhoac = dmax(u[0] * M.col, u[9] * M.col);
+    if (i >= 2 && i < M.ix - 2 && j >= 2 && j < M.jx - 2) r.dtc = dmin(r.dtc, dtc);
+    r.rhoac = dmax(r.rhoac, dmax(u[0] * M.col, u[9] * M.col));
 #pragma unroll
     for (int n = 0; n < 14; n++) U[n * N + k] = u[n];
   }
-  block_reduce_store<256, false>(r, 0, k < N, scs[m].red, red_lds);
+  block_reduce_store<256, false>(r, 0, true, scs[m].red, red_lds);
 }
 
 __global__ void __launch_bounds__(256) k_lock_init2(EnsArgs e, DevScalars* scs) {

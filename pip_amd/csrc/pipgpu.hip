@@ -1575,6 +1575,11 @@ static int ens_kernels_1d(pip_ens* e, EnsKernels* K) {
 
 // The kernels of 2-D members (16x15 tiles).
 constexpr int kGridY = 65535;  // limit of a grid's second dimension
+// Workgroups of a start launch: (as many as the largest member has 256 cells) x
+// members, but not more than these or 16 a member, since those past a small
+// member's cells only start and end (20,000 members of 16^2 and one of 1024^2:
+// 165 million of them, 37 of 48 ms).
+constexpr int kStartGroups = 65536;
 static int ens_kernels_2d(pip_ens* e, EnsKernels* K) {
   const size_t lds_stage = sizeof(double) * (size_t)TileGeom<2, 9, kEns2TX, kEns2TY>::LDS_DOUBLES;
   static bool attr = false;
@@ -1590,7 +1595,7 @@ static int ens_kernels_2d(pip_ens* e, EnsKernels* K) {
   const int n = e->n;
   long long cells = 0;  // of the largest member
   for (const EnsMember& M : e->hmem) cells = std::max(cells, (long long)M.ix * M.jx);
-  const unsigned nb = (unsigned)((cells + 255) / 256);
+  const unsigned nb = (unsigned)std::min((cells + 255) / 256, (long long)std::max(16, kStartGroups / n));
   K->start = [=](const EnsArgs& a) {
     for (int m0 = 0; m0 < n; m0 += kGridY) {  // at most kGridY members a launch
       EnsArgs b = a;
