@@ -422,8 +422,9 @@ struct TileBounded {
 // (1,3,2,4,5) (HLL_rot.f90:414-434, 315-325).  Bounded tiles run
 // hlld_flux_b / hllc_flux_b; the general functions take the faces these do
 // not cover and the tiles that are not bounded.  Measured on faces of a smooth
-// flow (1M faces, two 256-thread workgroups per CU): reconstruction 5.0 -> 4.0,
-// HLLD 20.6 -> 16.4, HLLC 11.9 -> 6.9 ps per face, the same bits.
+// flow (1M faces, two 256-thread workgroups per CU): reconstruction 5.0 -> 4.0
+// (with an fma for every half slope, see face_states), HLLD 20.6 -> 16.4, HLLC
+// 11.9 -> 6.9 ps per face, the same values.
 template <int FL, int NV, int DIR, int ST, int PV, int PF, bool BOUNDED = true>
 __device__ __forceinline__ void face_flux(const double* v, double* f, const Phys& ph, double cmax, bool bounded) {
   constexpr int NFL = FL ? 5 : NV;

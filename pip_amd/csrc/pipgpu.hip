@@ -234,7 +234,9 @@ static int launch_split_t(pip_ctx* c, const StageArgs& a) {
 // tiles) 11.5 / 13.3, 14.6 / 16.4, 16.5 / 18.2; 160^2 (230, 110) 11.9 / 14.8,
 // 14.9 / 16.5, 16.6 / 18.3; 240^2 (525, 240) 22 / 29, 15.2 / 17.0, 16.9 / 18.6;
 // 300^2 (817, 380) 28 / 36, 23.7 / 27.5, 22.1 / 24.8.  1-D, 127-cell split
-// against 255-cell one-pass tiles: 1024 cells 9.7 / 11.2, 11.7 / 13.7.
+// against 255-cell one-pass tiles: 1024 cells 9.7 / 11.2, 11.7 / 13.7; a whole
+// step of 256 to 24,000 cells 14 to 15 against 21 to 24 us, of 32,512 cells (256
+// split tiles) 15.4, of 32,513 (128 one-pass ones) 22.3.
 constexpr long long kCUs = 256;
 static bool one_round(int nx, int ny, int tx, int ty) {
   return (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) <= kCUs;
@@ -546,7 +548,10 @@ int pip_create(const pip_cfg* cfg, pip_ctx** out) {
   // halo that they read more of is in L2.  us per step, 16x15 and 16x7:
   // Orszag-Tang 1024^2 265 / 266, 1500^2 603 / 582, 2048^2 1109 / 1056; KH + IR
   // 1200^2 475 / 469, 2048^2 1346 / 1303.  Below, the last round decides
-  // (Orszag-Tang 400^2 60 / 69).
+  // (Orszag-Tang 400^2 60 / 69).  Relaxed arithmetic and the fluid-by-fluid
+  // kernel start the same way: relaxed, Orszag-Tang 64^2 29.1 / 27.2, 160^2 29.2 /
+  // 26.8, KH + IR 2048^2 1206 / 1139; both stages fluid by fluid 38.1 / 35.9, 38.5 /
+  // 35.6, 1625 / 1698 (row-major 16x15 tiles 1777).
   if (cfg->ndim == 2 && (long long)((c->nx + 15) / 16) * ((c->ny + 14) / 15) > 16 * 2 * kCUs) c->ty = 7;
   // by the 16x7 (127-cell) tiles, whatever tile is set: the set count is fixed
   // for the context
