@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import json
 import os
+import time
 
 from . import build
 
@@ -46,6 +47,21 @@ def stage_key(cfg, arith: str = "exact") -> str:
     return key if arith == "exact" else key + ":" + arith
 
 
+# The clock of a GPU that has idled (while a candidate was made) rises over the
+# first 25 to 30 ms of work: Orszag-Tang 1024^2 took 300 us a step there and 262
+# after, KH + IR 2048^2 1370 and 1290, and tiles 2 % apart changed places.
+WARM_S = 0.05
+
+
+def _warm(solver):
+    end = time.perf_counter() + WARM_S
+    while True:
+        solver.enqueue(3)
+        solver.sync()
+        if time.perf_counter() >= end:
+            return
+
+
 def two_pass_ok(cfg) -> bool:
     """Configurations the fluid-by-fluid stage kernel covers."""
     return cfg.ndim == 2 and cfg.flag_col == 1 and cfg.flag_pip_imp == 0
@@ -72,8 +88,7 @@ def tune_stage(make_solver, cfg, steps: int = 20, use_cache: bool = True, arith:
                   for m in sorted({1 << (cfg.t_order - 1), full})]
     for cand in cands:
         s = make_solver(cand)
-        s.enqueue(3)
-        s.sync()
+        _warm(s)
         ev = s.time_steps(steps, stages=False)
         timings["x".join(str(v) for v in cand)] = ev["total_ms"] / steps
         s.close()
